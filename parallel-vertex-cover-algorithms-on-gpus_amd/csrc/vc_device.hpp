@@ -37,9 +37,10 @@ static_assert(__builtin_offsetof(GDesc, n) == 0 && __builtin_offsetof(GDesc, off
 // Mutable search state of one graph (one 64-byte line, so graphs do not
 // share lines).
 struct GState {
+    // best and stop are read together (one 8-byte load per look)
     int32_t best;         // MVC incumbent; starts at U (src/main.cu:73 with VC 1)
-    uint32_t found;       // PVC: a cover <= k was found (kFound_d, src/main.cu:249-251)
     uint32_t stop;        // 1 = drop remaining work (found or budget exhausted)
+    uint32_t found;       // PVC: a cover <= k was found (kFound_d, src/main.cu:249-251)
     uint32_t outstanding; // live subtrees: queued items + owned by a worker
     uint64_t nodes;       // tree nodes spent on this graph
     uint32_t cover_lock;
@@ -142,6 +143,11 @@ struct SolveArgs {
     uint32_t lcap;          // mark-list capacity per worker (multiple of 4)
     uint32_t ncap;          // capacity of each rule-candidate list (multiple of 4)
     uint32_t mwords;        // mark-bitset words per worker (multiple of 4)
+    uint32_t xs_bytes;      // bytes of apply scratch and candidate lists per worker
+    uint32_t bits_max;      // nodes of at most this many live vertices go to the bitset search
+    uint32_t bits_lds;      // LDS bytes of one worker's contexts (vc_bits.hpp)
+    uint32_t ctx_bytes;     // bytes of one worker's published contexts
+    char *ctx;              // [workers][ctx_bytes] published contexts
     uint32_t worker_bytes;  // bytes of per-worker node storage (LDS or HBM)
     uint32_t depth;         // stack slots per worker
     uint32_t qsize;         // power of two
@@ -176,6 +182,10 @@ struct SolveArgs {
     // nearly all busy (0 = every worker starts at once)
     uint32_t active0;
     uint64_t dormant_ticks;
+    // bitset searches look at the graph's and the launch's shared words at
+    // every node (0) or every poll_mask + 1 nodes: with thousands of workers
+    // these reads contend on a handful of lines
+    uint32_t poll_mask;
     // node-budget flushes: workers per graph, the least number of workers
     // assumed to share a graph (vcg::flush_interval)
     uint32_t flush_share;

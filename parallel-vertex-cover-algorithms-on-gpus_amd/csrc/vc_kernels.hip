@@ -27,6 +27,8 @@
 // on blockDim, src/helperFunctions.cuh:453-478).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "vcgpu.h"
 #include "vc_bound.hpp"
 #include "vc_device.hpp"
@@ -272,6 +274,10 @@ template <typename DegT> constexpr uint32_t node_bytes_per_vertex()
     return sizeof(DegT) == 2 ? 8u : 16u;
 }
 
+//
+// Every function that works on a Node is inlined into the kernel: called, it
+// takes the Node by address and reloads its pointers from scratch memory (a
+// one-wave scan of 24,000 vertices took 4.3 instead of 3.1 ms).
 template <typename DegT, bool HBM, bool OFF16 = false, bool ADJ = false>
 struct Node {
     static constexpr bool kPacked = sizeof(DegT) == 2;
@@ -585,7 +591,7 @@ __device__ __forceinline__ void apply_one(const N &w, uint32_t u0, Cands &c)
 }
 
 template <class N>
-__device__ void apply_list(const N &w, uint32_t L, Cands &c)
+__device__ __forceinline__ void apply_list(const N &w, uint32_t L, Cands &c)
 {
     L = uni(L);
     w.sync();
@@ -662,6 +668,7 @@ __device__ void apply_list(const N &w, uint32_t L, Cands &c)
 // mark anything.
 struct Lanes {
     int s;        // sum of live degrees
+    int c;        // vertices of degree 1 or more
     int md;       // max degree of the lane's vertices
     uint32_t mv;  // lowest index with degree md in the lane
 };
@@ -669,6 +676,7 @@ struct Lanes {
 __device__ __forceinline__ void lanes_reset(Lanes &st)
 {
     st.s = 0;
+    st.c = 0;
     st.md = 0;
     st.mv = kNone;
 }
@@ -677,7 +685,10 @@ __device__ __forceinline__ void lanes_reset(Lanes &st)
 // index of the maximum (src/Sequential.cpp:50-58).
 __device__ __forceinline__ void lanes_add(Lanes &st, int dv, uint32_t v)
 {
-    if (dv > 0) st.s += dv;
+    if (dv > 0) {
+        st.s += dv;
+        ++st.c;
+    }
     if (dv > st.md) {
         st.md = dv;
         st.mv = v;
@@ -707,7 +718,7 @@ __device__ __forceinline__ uint32_t leaf_mark(const N &w, uint32_t v, uint32_t n
 }
 
 template <class N>
-__device__ uint32_t rule_leaf(const N &w, Cands &c)
+__device__ __forceinline__ uint32_t rule_leaf(const N &w, Cands &c)
 {
     uint32_t total = 0;
     for (;;) {
@@ -816,7 +827,7 @@ __device__ __forceinline__ void triangle_at(const N &w, uint32_t v, int dv, type
 // finds every triangle a full scan would.  A pass whose marks hit the list
 // capacity (the unmarked rest stays unexamined) makes the next pass full.
 template <class N>
-__device__ uint32_t rule_triangle(const N &w, Cands &c)
+__device__ __forceinline__ uint32_t rule_triangle(const N &w, Cands &c)
 {
     uint32_t total = 0;
     for (;;) {
@@ -875,7 +886,7 @@ __device__ uint32_t rule_triangle(const N &w, Cands &c)
 // w.list, at most lcap; the rest are found by the next scan).  When nothing
 // is marked, st describes the node exactly.
 template <class N>
-__device__ uint32_t scan_high(const N &w, uint32_t d, uint32_t T, Lanes &st)
+__device__ __forceinline__ uint32_t scan_high(const N &w, uint32_t d, uint32_t T, Lanes &st)
 {
     uint32_t L = 0;
     lanes_reset(st);
@@ -897,6 +908,7 @@ __device__ uint32_t scan_high(const N &w, uint32_t d, uint32_t T, Lanes &st)
 
 struct Summary {
     uint32_t edges;  // live edges (findNumOfEdges, src/helperFunctions.cuh:483-504)
+    uint32_t live;   // vertices with a live edge
     int32_t maxdeg;  // findMaxDegree (src/helperFunctions.cuh:450-481)
     uint32_t maxv;   // lowest index of maximum degree
 };
@@ -914,7 +926,7 @@ struct Summary {
 // do).  Returns the new cover size and, in *sum, the node's edge count and
 // max-degree vertex.
 template <class N>
-__device__ uint32_t reduce_node(const N &w, uint32_t d, uint32_t T, Summary *sum, Cands &c)
+__device__ __forceinline__ uint32_t reduce_node(const N &w, uint32_t d, uint32_t T, Summary *sum, Cands &c)
 {
     Lanes st;
     for (;;) {
@@ -931,15 +943,54 @@ __device__ uint32_t reduce_node(const N &w, uint32_t d, uint32_t T, Summary *sum
     }
     const int md = wave_max(st.md);
     sum->edges = (uint32_t)wave_sum(st.s) / 2u;
+    sum->live = (uint32_t)wave_sum(st.c);
     sum->maxdeg = md;
     sum->maxv = wave_min_u32((st.md == md && md > 0) ? st.mv : kNone);
     return d;
 }
 
+// More edges than `room` vertices can cover?  No `room` vertices cover more
+// edges than the sum of the `room` largest degrees, which is the sum over
+// the degrees x of min(room, vertices of degree x or more): one LDS histogram
+// (degrees of 63 and more in one entry) and a suffix sum over the lanes.
+// On ER n = 140, mean degree 9, it leaves a third of the tree that
+// bound_prunes' square alone visits (a BA n = 400, m = 4: half).  Node state
+// in HBM takes the maximum degree for every vertex: there the histogram's pass
+// would cost as much as the scan for the statistics.
+constexpr uint32_t kHistMaxN = 1024;
+template <class N>
+__device__ bool degrees_prune(const N &w, const Summary &s, uint32_t room)
+{
+    const uint32_t md = (uint32_t)s.maxdeg;
+    if ((uint64_t)s.edges > (uint64_t)room * md) return true;
+    if constexpr (N::kHbm) {
+        return false;
+    } else {
+        if (uni(w.n) > kHistMaxN) return false;
+        const uint32_t lane = lane_id();
+        w.xs[lane] = 0;
+        w.sync();
+        for (uint32_t base = 0, nv = uni(w.n); base < nv; base += 2u * kWave) {
+            const uint32_t v0 = base + 2u * lane;
+            int d0, d1;
+            w.pair(v0, nv, d0, d1);
+            if (d0 > 0) __hip_atomic_fetch_add(&w.xs[min(d0, 63)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            if (d1 > 0) __hip_atomic_fetch_add(&w.xs[min(d1, 63)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        }
+        w.sync();
+        const int h = w.xs[lane];
+        const int incl = wave_incl_scan(h);
+        const int ge = __builtin_amdgcn_readlane(incl, 63) - incl + h;  // degree `lane` or more
+        int cap = lane == 0u ? 0 : min(ge, (int)room);
+        if (lane == 63u && md > 63u) cap *= (int)(md - 62u);
+        return s.edges > (uint32_t)wave_sum(cap);
+    }
+}
+
 // Left child in place: v into the cover (deleteMaxDegreeVertex,
 // src/helperFunctions.cuh:200-215).
 template <class N>
-__device__ void take_vertex(const N &w, uint32_t v, Cands &c)
+__device__ __forceinline__ void take_vertex(const N &w, uint32_t v, Cands &c)
 {
     w.sync();
     if (lane_id() == 0) w.remove(v);
@@ -965,7 +1016,7 @@ __device__ void take_vertex(const N &w, uint32_t v, Cands &c)
 // rounds of at most lcap vertices.  Returns how many vertices were added
 // (deg(v) before the call).
 template <class N>
-__device__ uint32_t take_neighbours(const N &w, uint32_t v, Cands &c)
+__device__ __forceinline__ uint32_t take_neighbours(const N &w, uint32_t v, Cands &c)
 {
     uint32_t total = 0;
     const uint32_t b = w.off(v), e = w.off(v + 1);
@@ -991,7 +1042,7 @@ __device__ uint32_t take_neighbours(const N &w, uint32_t v, Cands &c)
 // Root node of a graph: its degrees, and the sketch sums over every
 // neighbour (all are live).  Padding vertices [n, npad) are in the cover.
 template <class N>
-__device__ void init_root(const N &w, const int32_t *deg0, uint32_t npad)
+__device__ __forceinline__ void init_root(const N &w, const int32_t *deg0, uint32_t npad)
 {
     using S2 = typename N::s2_t;
     for (uint32_t v = lane_id(); v < npad; v += kWave) {
@@ -1187,12 +1238,12 @@ __device__ __forceinline__ uint32_t copy_bytes(uint32_t cnt)
 // broker worklist (src/BWDWorkList.cuh) with 64-bit ring positions
 // ---------------------------------------------------------------------------
 
-// Writes one subtree (degrees at src, cover size d, pending branch vertex v
-// of graph g) into the ring if the occupancy guard admits it.  The caller
-// has already decided that a donation is wanted.
-template <class N>
-__device__ bool try_enqueue(const SolveArgs &a, const N &w, const char *src, uint32_t g, uint32_t d, uint32_t v,
-                            uint32_t slot_bytes)
+// Reserves a ring slot if the occupancy guard admits one more item (the
+// caller has already decided that a donation is wanted), and counts the
+// donated subtree as one more outstanding unit of graph g.  The caller then
+// writes the slot's data and its (g, d, v, kind) with agent-coherent stores and
+// calls publish_slot.
+__device__ __forceinline__ bool reserve_slot(const SolveArgs &a, uint32_t g, uint32_t &slot_out, uint32_t &ticket_out)
 {
     uint32_t ok = 0, slot = 0, ticket = 0;
     if (lane_id() == 0) {
@@ -1220,27 +1271,82 @@ __device__ bool try_enqueue(const SolveArgs &a, const N &w, const char *src, uin
     }
     ok = uni(ok);
     if (!ok) return false;
-    slot = uni(slot);
-    ticket = uni(ticket);
+    slot_out = uni(slot);
+    ticket_out = uni(ticket);
     handoff_observe();
-    copy_state_to_ring<N>(slot_rsrc(static_cast<char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes), src, a.npad,
-                          w.n);
-    if (lane_id() == 0) {
-        const u32x4 m = {g, d, v, 0u};
+    return true;
+}
+
+__device__ __forceinline__ void publish_slot(const SolveArgs &a, uint32_t slot, uint32_t ticket, u32x4 m)
+{
+    if (lane_id() == 0)
         __builtin_amdgcn_raw_buffer_store_b128(m, slot_rsrc(&a.q_meta[slot], 16u), 0u, 0, kCoherent);
-    }
     handoff_publish();
     if (lane_id() == 0) {
         st_rlx(&a.tickets[slot], ticket + 1u);
         fetch_add(&a.glob->counter, kEnqOne);
     }
+}
+
+// Writes one subtree (node state at src, cover size d, pending branch vertex v
+// of graph g) into the ring.
+template <class N>
+__device__ bool try_enqueue(const SolveArgs &a, const N &w, const char *src, uint32_t g, uint32_t d, uint32_t v,
+                            uint32_t slot_bytes)
+{
+    uint32_t slot, ticket;
+    if (!reserve_slot(a, g, slot, ticket)) return false;
+    copy_state_to_ring<N>(slot_rsrc(static_cast<char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes), src, a.npad,
+                          w.n);
+    publish_slot(a, slot, ticket, u32x4{g, d, v, 0u});
     return true;
 }
 
-// Takes one item if the occupancy guard says one is there.  On success the
-// degree array is in the worker's node storage and (g, d, v) are returned.
+// The same for a subtree of the bitset search (vc_bits.hpp) at context `ctx`:
+// word i < words of its masks in lane i.
+__device__ __forceinline__ bool try_enqueue_bits(const SolveArgs &a, uint32_t g, uint32_t d, uint32_t ctx, uint32_t words,
+                                                 uint32_t word, uint32_t slot_bytes)
+{
+    uint32_t slot, ticket;
+    if (!reserve_slot(a, g, slot, ticket)) return false;
+    if (lane_id() < words)
+        __builtin_amdgcn_raw_buffer_store_b32(word, slot_rsrc(static_cast<char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes),
+                                              4u * lane_id(), 0, kCoherent);
+    publish_slot(a, slot, ticket, u32x4{g, d, words, ctx + 1u});
+    return true;
+}
+
+// A worker's random numbers (a linear congruential generator): spread the
+// reactions of many workers to the same shared word.
+__device__ __forceinline__ uint32_t next_random(uint32_t &state)
+{
+    state = state * 1664525u + 1013904223u;
+    return state >> 16;
+}
+
+// Should this worker donate, given the launch's counter?  While workers wait
+// and the worklist holds fewer items than there are waiting workers (and
+// fewer than the -t threshold).  Of the many busy workers that see the same
+// shortage only about twice as many as items are missing act on it: when all
+// did, a search of 470,000 nodes on 4,096 workers made 183,000 donations and
+// took 48 ms, against 17 ms on 1,024 workers.
+__device__ __forceinline__ bool wants_donation(const SolveArgs &a, unsigned long long counter, uint32_t &rnd)
+{
+    const uint32_t lo = uni((uint32_t)counter), enq = uni((uint32_t)(counter >> 32));
+    const uint32_t waiting = lo & 0xFFFFu, busy = (lo >> 16) - waiting;
+    if (waiting == 0u || enq >= waiting || enq >= a.qthreshold) return false;
+    const uint32_t missing = waiting - enq;
+    if (2u * missing >= busy) return true;
+    return ((next_random(rnd) * busy) >> 16) < 2u * missing;
+}
+
+// Takes one item if the occupancy guard says one is there.  On success
+// (g, d, v) are returned and either the node state is in the worker's node
+// storage (ctx = kNone), or the item is a subtree of the bitset search of
+// context ctx: word i < v of its masks in lane i of `word`.
 template <bool SERVE, class N>
-__device__ bool try_dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_t &d, uint32_t &v, uint32_t slot_bytes)
+__device__ bool try_dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_t &d, uint32_t &v, uint32_t &ctx,
+                            uint32_t &word, uint32_t slot_bytes)
 {
     uint32_t ok = 0, slot = 0, ticket = 0;
     if (lane_id() == 0 && ld_rlx(&a.glob->count) > 0) {
@@ -1278,7 +1384,14 @@ __device__ bool try_dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_
     g = uni(m.x);
     d = uni(m.y);
     v = uni(m.z);
-    if constexpr (N::kPacked && !N::kHbm)
+    ctx = uni(m.w) - 1u;
+    word = 0;
+    if (ctx != kNone) {
+        if (lane_id() < v)
+            word = __builtin_amdgcn_raw_buffer_load_b32(
+                slot_rsrc(static_cast<const char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes), 4u * lane_id(), 0,
+                kCoherent);
+    } else if constexpr (N::kPacked && !N::kHbm)
         copy_state_to_lds<N, true>(w.base, static_cast<const char *>(a.q_deg) + (size_t)slot * slot_bytes, a.npad,
                                    uni(a.gdesc[g].n));
     else
@@ -1312,9 +1425,9 @@ __device__ void write_cover(const SolveArgs &a, const N &w, const GDesc &gd)
     }
 }
 
-// A cover of size d was reached (maxDegree == 0).
-template <class N>
-__device__ void record_cover(const SolveArgs &a, const N &w, const GDesc &gd, uint32_t g, uint32_t d)
+// A cover of size d was reached (maxDegree == 0); `write` stores its bitmap.
+template <class F>
+__device__ __forceinline__ void record_cover(const SolveArgs &a, const GDesc &gd, uint32_t g, uint32_t d, F &&write)
 {
     GState *gs = &a.gstate[g];
     if (gd.instance == 0) {
@@ -1342,7 +1455,7 @@ __device__ void record_cover(const SolveArgs &a, const N &w, const GDesc &gd, ui
                 fence_acq();
                 int cur = (int)uni((uint32_t)ld_rlx(&gs->best));
                 if (cur == (int)d) {
-                    write_cover(a, w, gd);
+                    write();
                     if (lane_id() == 0) st_rlx(&gs->cover_size, (int32_t)d);
                 }
                 fence_rel();
@@ -1356,7 +1469,7 @@ __device__ void record_cover(const SolveArgs &a, const N &w, const GDesc &gd, ui
             uint32_t first = 0;
             if (lane_id() == 0) first = atomicCAS(&gs->found, 0u, 1u) == 0u;
             if (uni(first)) {
-                write_cover(a, w, gd);
+                write();
                 if (lane_id() == 0) st_rlx(&gs->cover_size, (int32_t)d);
                 fence_rel();
             }
@@ -1394,19 +1507,17 @@ __device__ __forceinline__ uint32_t flush_interval(const SolveArgs &a, const GDe
 
 // Adds the nodes spent on graph g since the last flush to its count (and
 // stops it at its budget), and the HBM bytes of the slot copies made for it
-// (bytes_per_copy each) to the launch total.  Returns the next flush
-// interval when there was something to add.
+// to the launch total.  Returns the next flush interval when there was
+// something to add.
 template <bool kByWorkers>
 __device__ __forceinline__ void flush_nodes(const SolveArgs &a, const GDesc &gd, uint32_t g, uint64_t &pending,
-                                            uint32_t &copies, uint32_t bytes_per_copy, uint32_t &flush_every,
-                                            bool unit_end)
+                                            uint32_t &moved, uint32_t &flush_every, bool unit_end)
 {
     // copy bytes go to one launch-wide word: added at the end of a unit or
-    // every 256 copies, not at every (near a budget, frequent) node flush
-    if (unit_end || copies >= 256u) {
-        if (lane_id() == 0 && copies != 0u)
-            fetch_add(&a.glob->state_bytes, (unsigned long long)copies * bytes_per_copy);
-        copies = 0;
+    // after a megabyte, not at every (near a budget, frequent) node flush
+    if (unit_end || moved >= (1u << 20)) {
+        if (lane_id() == 0 && moved != 0u) fetch_add(&a.glob->state_bytes, (unsigned long long)moved);
+        moved = 0;
     }
     if (pending == 0) return;
     uint32_t next = 0;
@@ -1540,6 +1651,7 @@ __device__ __forceinline__ uint32_t roots_available(const SolveArgs &a)
 // 0 = terminate, 1 = queued item (degrees already in node storage), 2 = root.
 struct Acquired {
     uint32_t kind, g, d, v, root;
+    uint32_t ctx, word;  // a subtree of the bitset search (try_dequeue), else ctx = kNone
 };
 
 // Work for an idle worker: a queued subtree (kind 1), a root (kind 2: a
@@ -1558,9 +1670,9 @@ struct Acquired {
 // worker's claim attempt on the same words cost more than the search of a
 // small graph.
 template <bool SERVE, class N>
-__device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes, bool counted, uint32_t rid)
+__device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes, bool counted, uint32_t rid, uint32_t rnd)
 {
-    Acquired r = {0u, kNone, 0u, kNone, 0u};
+    Acquired r = {0u, kNone, 0u, kNone, 0u, kNone, 0u};
     // A cancelled or late launch hands out no more work.  Checked on every
     // call, not only when the worklist is empty: a worker that cycles
     // through queued units shorter than kFlushEvery nodes never reaches the
@@ -1571,18 +1683,28 @@ __device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes,
     if (!counted && lane_id() == 0) fetch_add(&a.glob->counter, kWaitOne);
     uint32_t spins = 0;
     for (;;) {
-        if (a.version == 1) {
-            uint32_t g, d, v;
-            if (try_dequeue<SERVE>(a, w, g, d, v, slot_bytes)) {
+        // One poll is one read of the termination word: items (batch: and
+        // roots) are there only when its "enqueued" field says so, and with
+        // fewer items than waiting workers only about twice as many workers
+        // as items try to take one.
+        const unsigned long long seen = ld_rlx(&a.glob->counter);
+        const uint32_t lo = uni((uint32_t)seen), hi = uni((uint32_t)(seen >> 32));
+        const uint32_t waiting = lo & 0xFFFFu, reg = lo >> 16;
+        const bool attempt = hi != 0u && (2u * hi >= waiting || ((next_random(rnd) * waiting) >> 16) < 2u * hi);
+        if (a.version == 1 && attempt) {
+            uint32_t g, d, v, ctx, word;
+            if (try_dequeue<SERVE>(a, w, g, d, v, ctx, word, slot_bytes)) {
                 r.kind = 1;
                 r.g = g;
                 r.d = d;
                 r.v = v;
+                r.ctx = ctx;
+                r.word = word;
                 return r;
             }
         }
         if constexpr (!SERVE) {
-            if ((rid < a.roots || spins >= 2u) && uni(ld_rlx(&a.glob->next_root)) < a.roots) {
+            if (hi != 0u && (rid < a.roots || spins >= 2u) && uni(ld_rlx(&a.glob->next_root)) < a.roots) {
                 uint32_t idx = kNone;
                 if (lane_id() == 0) {
                     idx = fetch_add(&a.glob->next_root, 1u);
@@ -1629,10 +1751,6 @@ __device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes,
                 }
             }
         }
-        unsigned long long c = 0;
-        if (lane_id() == 0) c = ld_rlx(&a.glob->counter);
-        uint32_t lo = uni((uint32_t)c), hi = uni((uint32_t)(c >> 32));
-        uint32_t waiting = lo & 0xFFFFu, reg = lo >> 16;
         // batch: unclaimed roots are in `hi`; serving: no root is coming once
         // the host has shut down and every published request is taken
         bool no_more_roots = true;
@@ -1643,9 +1761,10 @@ __device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes,
             if (lane_id() == 0) st_rlx(&a.glob->done_flag, 1u);
             return r;
         }
-        if (uni(ld_rlx(&a.glob->done_flag)) || uni(ld_rlx(&a.glob->cancel))) return r;
-        if (lane_id() == 0) late = past_deadline(a);
-        if (uni(late)) return r;
+        if ((spins & 3u) == 3u) {
+            if (lane_id() == 0) late = ld_rlx(&a.glob->done_flag) | ld_rlx(&a.glob->cancel) | (uint32_t)past_deadline(a);
+            if (uni(late)) return r;
+        }
         backoff_idle(++spins, a.idle_cap, waiting);
     }
 }
@@ -1753,6 +1872,12 @@ __device__ __forceinline__ GDesc load_desc(const GDesc *p)
     return d;
 }
 
+}  // namespace vcg
+
+#include "vc_bits.hpp"
+
+namespace vcg {
+
 // ---------------------------------------------------------------------------
 // the persistent solve kernel
 // ---------------------------------------------------------------------------
@@ -1770,10 +1895,13 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     if constexpr (STAGED)
         if (wid >= a.active0 && !dormant_join(a, wid)) return;
 
+    // LDS: the contexts of every worker's bitset searches, then (LDS variants)
+    // the node storage
+    const BitsLds bits_lds = {reinterpret_cast<char *>(smem4) + (size_t)wib * a.bits_lds};
     // node storage: node state (npad * node_bytes_per_vertex) | list [lcap u32] | mark [mwords u32] |
-    // xs [64 i32] | cand [npad]; a stack or worklist slot holds the node state
+    // xs [64 i32], cand, cand3 (xs_bytes in all); a stack or worklist slot holds the node state
     char *store = HBM ? a.hbm_nodes + (size_t)wid * a.worker_bytes
-                      : reinterpret_cast<char *>(smem4) + (size_t)wib * a.worker_bytes;
+                      : reinterpret_cast<char *>(smem4) + (size_t)(blockDim.x / kWave) * a.bits_lds + (size_t)wib * a.worker_bytes;
     const uint32_t slot_bytes = a.npad * node_bytes_per_vertex<DegT>();
     static_assert(!ADJ || OFF16, "the LDS adjacency sits after the LDS offsets");
     using NodeT = Node<DegT, HBM, OFF16, ADJ>;
@@ -1797,7 +1925,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     w.cand3 = w.cand + a.ncap;
     w.ncap = a.ncap;
     w.src = nullptr;
-    w.off16 = OFF16 ? reinterpret_cast<uint16_t *>(w.cand3 + a.ncap) : nullptr;
+    w.off16 = OFF16 ? reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(w.xs) + a.xs_bytes) : nullptr;
     // the adjacency follows the npad + 2 offset entries
     w.adj16 = ADJ ? w.off16 + a.npad + 2u : nullptr;
     w.dst = nullptr;
@@ -1834,13 +1962,16 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     Cands c;            // rule candidates listed since the last passes
     uint32_t off16_g = kNone;  // graph whose offsets the LDS copy holds
     uint64_t pending = 0, total_nodes = 0, idle_ticks = 0, donations = 0, steals = 0;
-    // slot copies of the current graph's node state since the last flush:
-    // stack pushes and pops, steals (ring slot in) and donations (stack slot
-    // to ring slot, two); flush_nodes adds their HBM bytes to the launch total
-    uint32_t copies = 0;
+    // HBM bytes of the node state moved since the last flush: stack pushes
+    // and pops, steals (ring slot in) and donations (stack slot to ring slot,
+    // two); flush_nodes adds them to the launch total
+    uint32_t moved = 0;
     uint32_t flush_every = kFlushEvery;  // see flush_interval
+    uint32_t rnd = wid * 2654435761u;    // random state (next_random)
 
     for (;;) {
+        // a subtree for the bitset search: its live vertices, or a donated one
+        uint32_t bits = 0, bits_ctx = kNone, bits_word = 0;
         if (!have) {
             if (top < bot) {
                 top = -1;
@@ -1855,7 +1986,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     copy_state_to_lds<NodeT>(w.base, stk + (size_t)ts * slot_bytes, a.npad, w.n);
                 else
                     copy_state<NodeT>(w.base, stk + (size_t)ts * slot_bytes, a.npad, w.n);
-                ++copies;
+                moved += copy_bytes<NodeT>(w.n);
                 w.sync();
                 d = uni(m.x);
                 uint32_t v = uni(m.y);
@@ -1866,20 +1997,19 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
             } else {
                 if (g != kNone) {
                     total_nodes += pending;
-                    flush_nodes<STAGED>(a, gd, g, pending, copies, copy_bytes<NodeT>(w.n), flush_every, true);
+                    flush_nodes<STAGED>(a, gd, g, pending, moved, flush_every, true);
                     finish_unit<SERVE>(a, g, gd);
                     g = kNone;
                 }
                 if (lane_id() == 0 && ld_rlx(&a.glob->cancel)) st_rlx(&a.glob->done_flag, 1u);
                 const uint64_t t_idle = wall_clock64();
-                Acquired q = acquire<SERVE>(a, w, slot_bytes, counted, rid);
+                Acquired q = acquire<SERVE>(a, w, slot_bytes, counted, rid, rnd ^ (uint32_t)t_idle);
                 counted = false;
                 idle_ticks += wall_clock64() - t_idle;
                 if (q.kind == 0) break;
                 steals += q.kind == 1;
                 if (q.kind == 1) {
                     g = q.g;
-                    copies = 1u;
                 } else {
                     g = a.version == 1 ? q.root : (q.root >> a.start_depth);
                 }
@@ -1892,7 +2022,8 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 }
                 w.n = gd.n;
                 w.src = a.gbuf + gd.off_src;
-                if (OFF16 && g != off16_g) {
+                if (q.kind == 1) moved = q.ctx == kNone ? copy_bytes<NodeT>(w.n) : 4u * q.v;
+                if (OFF16 && g != off16_g && q.ctx == kNone) {
                     // a graph this worker has not held last: its offsets into LDS
                     if constexpr (ADJ) {
                         // and its adjacency (2m entries, vertex ids below 2^15)
@@ -1907,7 +2038,12 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 }
                 w.dst = a.gbuf + gd.off_dst;
                 w.bits = gd.off_bits ? a.gbuf + gd.off_bits : nullptr;
-                if (q.kind == 1) {
+                if (q.ctx != kNone) {
+                    d = q.d;
+                    descend = 0;
+                    bits_ctx = q.ctx;
+                    bits_word = q.word;
+                } else if (q.kind == 1) {
                     d = q.d;
                     cands_reset(c, q.v == kNone);
                     if (q.v != kNone) d += take_neighbours(w, q.v, c);
@@ -1927,61 +2063,106 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
             }
         }
 
-        GState *gs = &a.gstate[g];
-        // the stop flag and the incumbent in flight together (one round
-        // trip to L2 per node instead of two)
-        const uint32_t stop_now = ld_rlx(&gs->stop);
-        const uint32_t best_now = (uint32_t)ld_rlx(&gs->best);
-        if (uni(stop_now)) {
-            // graph finished by someone else (PVC found, budget): drop local work
-            top = -1;
-            bot = 0;
-            have = false;
-            continue;
-        }
-        if (++pending >= flush_every) {
-            total_nodes += pending;
-            flush_nodes<STAGED>(a, gd, g, pending, copies, copy_bytes<NodeT>(w.n), flush_every, false);
-            uint32_t stop_all = 0;
-            if (lane_id() == 0) stop_all = ld_rlx(&a.glob->cancel) || past_deadline(a);
-            if (uni(stop_all)) {
+        GState *const gs = &a.gstate[g];
+        uint32_t v = kNone;
+        if (bits_ctx == kNone) {
+            // the stop flag and the incumbent in flight together (one round
+            // trip to L2 per node instead of two)
+            const unsigned long long state_now = ld_rlx(reinterpret_cast<unsigned long long *>(&gs->best));
+            const uint32_t stop_now = (uint32_t)(state_now >> 32), best_now = (uint32_t)state_now;
+            if (uni(stop_now)) {
+                // graph finished by someone else (PVC found, budget): drop local work
                 top = -1;
                 bot = 0;
                 have = false;
                 continue;
             }
-        }
+            if (++pending >= flush_every) {
+                total_nodes += pending;
+                flush_nodes<STAGED>(a, gd, g, pending, moved, flush_every, false);
+                uint32_t stop_all = 0;
+                if (lane_id() == 0) stop_all = ld_rlx(&a.glob->cancel) || past_deadline(a);
+                if (uni(stop_all)) {
+                    top = -1;
+                    bot = 0;
+                    have = false;
+                    continue;
+                }
+            }
 
-        const bool mvc = gd.instance == 0;
-        uint32_t T = mvc ? uni(best_now) : gd.k + 1u;
-        Summary s;
-        d = reduce_node(w, d, T, &s, c);
+            const bool mvc = gd.instance == 0;
+            uint32_t T = mvc ? uni(best_now) : gd.k + 1u;
+            Summary s;
+            d = reduce_node(w, d, T, &s, c);
 
-        // the live incumbent (another worker may have lowered it while the
-        // rules ran with T); the bound uses both (bound_prunes)
-        const uint32_t B = mvc ? uni((uint32_t)ld_rlx(&gs->best)) : T;
-        if (bound_prunes(s.edges, d, T, B)) {
-            have = false;
-            descend = 0;
-            continue;
-        }
-        if (s.maxdeg == 0) {
-            record_cover(a, w, gd, g, d);
-            have = false;
-            descend = 0;
-            continue;
-        }
-        const uint32_t v = s.maxv;
-        if (descend > 0) {
-            // static split: follow this worker's path bit (src/LocalStacks.cuh:121-157)
-            uint32_t bit = (path >> (a.start_depth - descend)) & 1u;
-            --descend;
-            if (bit == 0u) {
+            // the live incumbent (another worker may have lowered it while the
+            // rules ran with T); the bound uses both (bound_prunes)
+            const uint32_t B = mvc ? uni((uint32_t)ld_rlx(&gs->best)) : T;
+            if (bound_prunes(s.edges, d, T, B)) {
+                have = false;
+                descend = 0;
+                continue;
+            }
+            if (s.maxdeg == 0) {
+                record_cover(a, gd, g, d, [&] { write_cover(a, w, gd); });
+                have = false;
+                descend = 0;
+                continue;
+            }
+            if (degrees_prune(w, s, B - 1u - d)) {
+                have = false;
+                descend = 0;
+                continue;
+            }
+            v = s.maxv;
+            if (descend > 0) {
+                // static split: follow this worker's path bit (src/LocalStacks.cuh:121-157)
+                uint32_t bit = (path >> (a.start_depth - descend)) & 1u;
+                --descend;
+                if (bit == 0u) {
+                    take_vertex(w, v, c);
+                    d += 1;
+                } else {
+                    d += take_neighbours(w, v, c);
+                }
+                continue;
+            }
+            if (s.live <= a.bits_max) {
+                bits = s.live;
+            } else if (s.maxdeg <= 2) {
+                // cycles only: some minimum cover holds v
                 take_vertex(w, v, c);
                 d += 1;
-            } else {
-                d += take_neighbours(w, v, c);
+                continue;
             }
+        }
+        if (bits != 0u || bits_ctx != kNone) {
+            BitsWorker bw;
+            bw.stk = stk;
+            bw.stk_meta = stk_meta;
+            bw.slot_bytes = slot_bytes;
+            bw.wid = wid;
+            bw.top = top;
+            bw.bot = bot;
+            bw.pending = pending;
+            bw.total_nodes = total_nodes;
+            bw.donations = donations;
+            bw.moved = moved;
+            bw.flush_every = flush_every;
+            bw.d = d;
+            bw.home = bits_ctx;
+            bw.rnd = rnd;
+            const uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();  // a
+            bit_search<STAGED>(args, w, bits_lds, gd, g, bits, bits_word, bw);
+            top = bw.top;
+            bot = bw.bot;
+            pending = bw.pending;
+            total_nodes = bw.total_nodes;
+            donations = bw.donations;
+            moved = bw.moved;
+            flush_every = bw.flush_every;
+            rnd = bw.rnd;
+            have = false;
             continue;
         }
         // Branch: the right child (N(v) into the cover) is stored as its
@@ -1991,7 +2172,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         // (an entry pushed at cover size d sits at index <= d); a smaller
         // configured depth hands the oldest entry to the worklist instead.
         if (top - bot + 1 >= (int)a.depth) {
-            bool moved = false;
+            bool sent = false;
             if (a.version == 1) {
                 for (uint32_t spins = 0;; ++spins) {
                     const uint32_t bs = (uint32_t)bot % a.depth;
@@ -1999,8 +2180,8 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     if (try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(m.x), uni(m.y), slot_bytes)) {
                         ++bot;
                         ++donations;
-                        copies += 2u;
-                        moved = true;
+                        moved += 2u * copy_bytes<NodeT>(w.n);
+                        sent = true;
                         break;
                     }
                     uint32_t late = 0;
@@ -2009,7 +2190,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     backoff(spins < 4 ? spins : 4);
                 }
             }
-            if (!moved) {
+            if (!sent) {
                 // hybrid: the wait ended because the graph stopped or the
                 // launch is cancelled; stack-only: the depth is exact, so
                 // this is an internal error
@@ -2018,27 +2199,30 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 continue;
             }
         }
-        ++top;
-        const uint32_t ts = (uint32_t)top % a.depth;
-        copy_state<NodeT>(stk + (size_t)ts * slot_bytes, w.base, a.npad, w.n);
-        if (lane_id() == 0) stk_meta[ts] = make_uint2(d, v);
-        ++copies;
-        if (a.version == 1) {
-            // Donate while workers wait and the worklist holds fewer items
-            // than there are waiting workers (and fewer than the -t
-            // threshold).  The OLDEST local entry goes: it is the shallowest
-            // and so the largest subtree this worker holds.
-            unsigned long long c = 0;
-            if (lane_id() == 0) c = ld_rlx(&a.glob->counter);
-            int waiting = (int)(uni((uint32_t)c) & 0xFFFFu);
-            int enq = (int)uni((uint32_t)(c >> 32));
-            if (waiting > 0 && enq < waiting && enq < (int)a.qthreshold && top >= bot) {
+        // Donate while workers wait (wants_donation).  The OLDEST local entry
+        // goes: it is the shallowest and so the largest subtree this worker
+        // holds.  With an empty stack that is the right child itself, which
+        // then goes from the node storage straight to the worklist (a
+        // BA n = 2,000 search, a chain of nodes that each donate their
+        // right child, took 0.93 ms with the copy through the stack).
+        const bool donate = a.version == 1 && wants_donation(a, ld_rlx(&a.glob->counter), rnd);
+        if (donate && top < bot && uni(try_enqueue(a, w, w.base, g, d, v, slot_bytes)) != 0u) {
+            ++donations;
+            moved += copy_bytes<NodeT>(w.n);
+        } else {
+            const bool older = top >= bot;
+            ++top;
+            const uint32_t ts = (uint32_t)top % a.depth;
+            copy_state<NodeT>(stk + (size_t)ts * slot_bytes, w.base, a.npad, w.n);
+            if (lane_id() == 0) stk_meta[ts] = make_uint2(d, v);
+            moved += copy_bytes<NodeT>(w.n);
+            if (donate && older) {
                 const uint32_t bs = (uint32_t)bot % a.depth;
                 uint2 m = stk_meta[bs];
                 if (try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(m.x), uni(m.y), slot_bytes)) {
                     ++bot;
                     ++donations;
-                    copies += 2u;
+                    moved += 2u * copy_bytes<NodeT>(w.n);
                 }
             }
         }
@@ -2131,7 +2315,12 @@ __global__ void init_kernel(SolveArgs a, uint32_t units, uint32_t preload_roots)
         a.gstate[g] = s;
     }
     for (uint32_t i = tid; i < a.qsize; i += stride) a.tickets[i] = 0u;
-    for (uint32_t i = tid; i < a.workers; i += stride) a.wstats[i] = WorkerStats{};
+    for (uint32_t i = tid; i < a.workers; i += stride) {
+        a.wstats[i] = WorkerStats{};
+        // users of the worker's contexts
+        for (uint32_t l = 0; l < kCtxLevels; ++l)
+            reinterpret_cast<uint32_t *>(a.ctx + (size_t)i * a.ctx_bytes)[l] = 0u;
+    }
     if (tid == 0) {
         Global z = {};  // t0 = 0: the first solve worker to start sets it
         if (preload_roots) z.counter = (unsigned long long)a.roots * kEnqOne;
@@ -2210,12 +2399,12 @@ template __global__ void solve_kernel<int16_t, false, false>(SolveArgs);
 // candidate lists a worker's LDS at n = 400 lets 28 workers share a CU.
 // Measured per batched step: 2.87 s at 7 waves against 3.16 s at 6 (80
 // VGPRs) and 3.38 s at 8 (64 VGPRs, 68 spilled).
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void solve_kernel_off16(SolveArgs a)
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void solve_kernel_off16(SolveArgs a)
 {
     solve_body<int16_t, false, false, true, false>(a);
 }
 // The same with a staged start (launches with few roots, dormant_join).
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void solve_kernel_off16_staged(SolveArgs a)
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void solve_kernel_off16_staged(SolveArgs a)
 {
     solve_body<int16_t, false, false, true, true>(a);
 }
@@ -2223,7 +2412,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void 
 // launches of few graphs whose adjacency fits beside the node state (small
 // searches are chains of dependent rule passes, each waiting for adjacency
 // reads; from LDS those take ~100 cycles instead of an L2 or MALL trip).
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void solve_kernel_off16_adj(SolveArgs a)
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void solve_kernel_off16_adj(SolveArgs a)
 {
     solve_body<int16_t, false, false, true, true, true>(a);
 }
@@ -2452,13 +2641,13 @@ const void *kernel_of(int variant, bool serve, bool off16 = false, bool adj = fa
 
 struct Plan {
     int variant;
-    uint32_t npad, lcap, ncap, mwords, worker_bytes, deg_bytes, slot_bytes, wpb, block_dim, blocks_per_cu,
+    uint32_t npad, lcap, ncap, mwords, xs_bytes, bits_max, ctx_bytes, worker_bytes, deg_bytes, slot_bytes, wpb, block_dim, blocks_per_cu,
         num_blocks, workers;
     uint32_t depth, qsize, qthreshold, roots, units;
     uint32_t off16;  // workers keep their graph's srcPtr in LDS as uint16
     uint32_t adj;    // ... and its dst (solve_kernel_off16_adj, a staged launch)
     size_t smem;
-    size_t off_glob, off_stk, off_meta, off_qdeg, off_qmeta, off_tickets, off_wnodes, off_hbm, total;
+    size_t off_glob, off_stk, off_meta, off_qdeg, off_qmeta, off_tickets, off_wnodes, off_ctx, off_hbm, total;
 };
 
 // entries per rule-candidate list: small enough that 28 workers' LDS fits a
@@ -2492,16 +2681,29 @@ void size_storage(Plan &pl, uint32_t nmax, uint32_t deg_bytes, bool off16 = fals
     pl.ncap = std::min<uint32_t>(round_up(nmax, 4u), adj_entries ? kCandCapLarge : cand_cap);
     const uint32_t id_bytes = deg_bytes == 2u ? 2u : 4u;  // mark and candidate list entries
     pl.mwords = round_up((nmax + 31u) / 32u, 4u);
-    const uint32_t cand_bytes = 2u * pl.ncap * id_bytes;
+    // xs and the two candidate lists; vcg::build_rows keeps a byte per vertex there
+    pl.xs_bytes = std::max(4u * vcg::kWave + 2u * pl.ncap * id_bytes, round_up(pl.npad, 4u));
+    pl.ctx_bytes = vcg::kHbmCover + vcg::kCtxLevels * round_up(4u * round_up((nmax + 31u) / 32u, 2u), 128u);
     pl.worker_bytes =
-        round_up(pl.slot_bytes + id_bytes * pl.lcap + 4u * pl.mwords + 4u * vcg::kWave + cand_bytes +
+        round_up(pl.slot_bytes + id_bytes * pl.lcap + 4u * pl.mwords + pl.xs_bytes +
                      (off16 ? 2u * (pl.npad + 2u) : 0u) + 2u * round_up(adj_entries, 4u),
                  64u);
 }
 
+// LDS of a worker's contexts, and of a workgroup of wpb workers with their
+// node storage in LDS.
+uint32_t bits_lds(const Plan &pl) { return pl.bits_max == vcg::kBitsMax ? vcg::kCtxLdsBytes : vcg::kCtxLdsSmall; }
+size_t lds_bytes(const Plan &pl, uint32_t wpb) { return (size_t)wpb * (bits_lds(pl) + pl.worker_bytes); }
+
 // Launch shape shared by the batch solve and the server: node storage,
 // workgroup, grid from the occupancy query, worklist, and the memory plan.
 constexpr uint32_t kServeWorkersPerCU = 2;
+// One worker per SIMD: a bitset search is a chain of scalar and vector
+// instructions with next to no memory access, so one wave nearly fills its
+// SIMD's issue slots, and more workers only share the same subtrees in smaller
+// pieces (ER n = 186, mean degree 9.95, 450,000 nodes: 12.2 ms with 1,024
+// workers, 17.2 with 512, 26 with 1,792).
+constexpr uint32_t kSolveWorkersPerCU = 4;
 constexpr uint32_t kMaxBlockDim = 1024;   // the solve kernels' launch bound
 constexpr uint32_t kMaxWorkers = 0xFFFFu; // 16-bit worker counts in the termination word
 
@@ -2526,13 +2728,16 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     // -g 0 forbids it); int16 degrees while n < 32768 (VC_FLAG_WIDE forces
     // int32).
     const bool wide = nmax >= 32768u || (p->flags & VC_FLAG_WIDE) != 0u;
+    pl.bits_max = vcg::kBitsMax;
     size_storage(pl, nmax, wide ? 4u : 2u);
     uint32_t wpb = block_dim / vcg::kWave;
     bool hbm = wide || p->use_global_memory == 1;
     if (!hbm) {
         if (!p->block_dim)
-            while (wpb > 1 && (size_t)wpb * pl.worker_bytes > lds_limit) wpb /= 2;
-        hbm = (size_t)wpb * pl.worker_bytes > lds_limit;
+            while (wpb > 1 && lds_bytes(pl, wpb) > lds_limit) wpb /= 2;
+        // an explicit workgroup whose workers fit with smaller contexts only
+        if (lds_bytes(pl, wpb) > lds_limit) pl.bits_max = vcg::kBitsMaxSmall;
+        hbm = lds_bytes(pl, wpb) > lds_limit;
     }
     if (hbm && p->use_global_memory == 0) return VC_ENOTSUP;
     pl.variant = wide ? kHbm32 : hbm ? kHbm16 : kLds16;
@@ -2544,7 +2749,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     if (!serve && off16_ok && pl.variant == kLds16) {
         Plan t = pl;
         size_storage(t, nmax, 2u, true);
-        if ((size_t)wpb * t.worker_bytes <= lds_limit) {
+        if (lds_bytes(t, wpb) <= lds_limit) {
             pl = t;
             pl.off16 = 1u;
         }
@@ -2555,8 +2760,8 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
             size_storage(ta, nmax, 2u, true, adj_entries);
             uint32_t wa = wpb;
             if (!p->block_dim)
-                while (wa > 1 && (size_t)wa * ta.worker_bytes > lds_limit) wa /= 2;
-            if ((size_t)wa * ta.worker_bytes <= lds_limit) {
+                while (wa > 1 && lds_bytes(ta, wa) > lds_limit) wa /= 2;
+            if (lds_bytes(ta, wa) <= lds_limit) {
                 pl = ta;
                 pl.off16 = 1u;
                 pl.adj = 1u;
@@ -2566,7 +2771,8 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     }
     pl.wpb = wpb;
     pl.block_dim = wpb * vcg::kWave;
-    pl.smem = hbm ? 0 : (size_t)pl.wpb * pl.worker_bytes;
+    if (hbm) pl.bits_max = (size_t)wpb * vcg::kCtxLdsBytes <= lds_limit ? vcg::kBitsMax : vcg::kBitsMaxSmall;
+    pl.smem = (size_t)pl.wpb * (bits_lds(pl) + (hbm ? 0u : pl.worker_bytes));
     if (pl.smem > lds_limit) return VC_ENOTSUP;
 
     int bpc = 0;
@@ -2585,6 +2791,9 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
         // occupancy grid a vc_solve issued beside a server waited for it.
         auto_blocks = std::min<uint32_t>(
             auto_blocks, std::max<uint32_t>(1u, kServeWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
+    } else {
+        auto_blocks = std::min<uint32_t>(
+            auto_blocks, std::max<uint32_t>(1u, kSolveWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
     }
     pl.num_blocks = p->num_blocks ? p->num_blocks : auto_blocks;
     // the termination word counts waiting and registered workers in 16-bit
@@ -2626,6 +2835,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
         pl.off_qmeta = take((size_t)pl.qsize * sizeof(uint4));
         pl.off_tickets = take((size_t)pl.qsize * sizeof(uint32_t));
         pl.off_wnodes = take((size_t)pl.workers * sizeof(vcg::WorkerStats));
+        pl.off_ctx = take((size_t)pl.workers * pl.ctx_bytes);
         pl.off_hbm = take(pl.variant != kLds16 ? (size_t)pl.workers * pl.worker_bytes : 0);
         pl.total = off;
         if (pl.total <= budget || pl.num_blocks <= 1) break;
@@ -2693,6 +2903,11 @@ void fill_args(SolveArgs &a, const Plan &pl, char *base, uint32_t version, uint3
     a.lcap = pl.lcap;
     a.ncap = pl.ncap;
     a.mwords = pl.mwords;
+    a.xs_bytes = pl.xs_bytes;
+    a.ctx = base + pl.off_ctx;
+    a.ctx_bytes = pl.ctx_bytes;
+    a.bits_max = pl.bits_max;
+    a.bits_lds = bits_lds(pl);
     a.worker_bytes = pl.worker_bytes;
     a.depth = pl.depth;
     a.qsize = pl.qsize;
@@ -2726,11 +2941,11 @@ void launch_variant(const Plan &pl, hipStream_t stream, const SolveArgs &a)
             break;
         case kHbm16:
             hipLaunchKernelGGL((vcg::solve_kernel<int16_t, true, false, true>), dim3(pl.num_blocks),
-                               dim3(pl.block_dim), 0, stream, a);
+                               dim3(pl.block_dim), pl.smem, stream, a);
             break;
         default:
             hipLaunchKernelGGL((vcg::solve_kernel<int32_t, true, false, true>), dim3(pl.num_blocks),
-                               dim3(pl.block_dim), 0, stream, a);
+                               dim3(pl.block_dim), pl.smem, stream, a);
             break;
         }
         return;
@@ -2745,11 +2960,11 @@ void launch_variant(const Plan &pl, hipStream_t stream, const SolveArgs &a)
                                pl.smem, stream, a);
         break;
     case kHbm16:
-        hipLaunchKernelGGL((vcg::solve_kernel<int16_t, true, SERVE>), dim3(pl.num_blocks), dim3(pl.block_dim), 0,
+        hipLaunchKernelGGL((vcg::solve_kernel<int16_t, true, SERVE>), dim3(pl.num_blocks), dim3(pl.block_dim), pl.smem,
                            stream, a);
         break;
     default:
-        hipLaunchKernelGGL((vcg::solve_kernel<int32_t, true, SERVE>), dim3(pl.num_blocks), dim3(pl.block_dim), 0,
+        hipLaunchKernelGGL((vcg::solve_kernel<int32_t, true, SERVE>), dim3(pl.num_blocks), dim3(pl.block_dim), pl.smem,
                            stream, a);
         break;
     }
@@ -3009,6 +3224,7 @@ SolveArgs solve_args(const vc_ctx *ctx, const vc_graphs *set, const vc_params *p
     // deadline on the device wall clock (every wait loop checks it)
     const uint64_t ms = params->time_limit_ms ? params->time_limit_ms : 3600ull * 1000ull;
     fill_args(a, pl, base, params->version, params->start_depth, ms * (uint64_t)ctx->wall_khz);
+    a.poll_mask = 0u;
     a.flush_share = std::max<uint32_t>(1u, pl.workers / std::max<uint32_t>(1u, a.num_graphs));
     // staged start (vcg::dormant_join) when the grid is automatic and the
     // roots could keep fewer than half the workers busy; the adjacency

@@ -1,0 +1,49 @@
+"""The bitset search (remainders of at most 256 live vertices, vc_bits.hpp)
+at the sizes where its layout changes: one vertex below, at and above each
+context size (32, 48, 64, 96, 128 and 256 vertices; 64 K vertices fill K slots
+of a lane).  MVC, and PVC at k = MVC - 1 and MVC, against the CPU oracle; every
+cover is checked.  All answers are whole numbers: no tolerance."""
+import numpy as np
+import pytest
+
+import graphgen
+import oracle as O
+import vcgpu
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [s + d for s in (32, 48, 64, 96, 128, 256) for d in (-1, 0, 1)]
+
+
+def _graphs(n):
+    # no vertex of degree 0 to 2 at the root, so the first context has n vertices
+    out = [("dense", graphgen.erdos_renyi(n, 0.9, 4000 + n))]
+    if n <= 97:
+        out.append(("sparse", graphgen.erdos_renyi(n, 6.0 / n, 5000 + n)))
+    return out
+
+
+@pytest.mark.parametrize("version", [vcgpu.VC_HYBRID, vcgpu.VC_STACK_ONLY])
+@pytest.mark.parametrize("n", SIZES)
+def test_context_sizes_match_oracle(ctx, n, version):
+    params = vcgpu.Params(version=version, start_depth=2, time_limit_ms=60000)
+    for name, e in _graphs(n):
+        og = O.from_edges(n, e)
+        want, stats, _ = O.mvc(og, max_nodes=2_000_000)
+        assert stats["completed"], (name, n)
+        g = vcgpu.csr_from_edges(n, e)
+        gs = ctx.upload([g, g, g])
+        # U = n - 1 (any n - 1 vertices cover): the search has to find the cover itself
+        jobs = [vcgpu.Job(vcgpu.VC_MVC, 0, n - 1, 0), vcgpu.Job(vcgpu.VC_PVC, want - 1, n - 1, 0),
+                vcgpu.Job(vcgpu.VC_PVC, want, n - 1, 0)]
+        (mvc, no, yes), _, st = ctx.solve(gs, jobs, params)
+        assert st == vcgpu.VC_OK
+        assert mvc.solved and mvc.minimum == want, (name, n, mvc.minimum, want)
+        assert no.solved and not no.k_found, (name, n)
+        assert yes.solved and yes.k_found, (name, n)
+        for r in (mvc, yes):
+            if r.cover is None:
+                assert want == n - 1, (name, n)  # nothing smaller than U exists
+                continue
+            assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)), (name, n)
+            assert int(np.sum(r.cover)) == want, (name, n)
