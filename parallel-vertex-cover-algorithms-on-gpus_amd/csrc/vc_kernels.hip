@@ -2328,6 +2328,219 @@ __global__ void init_kernel(SolveArgs a, uint32_t units, uint32_t preload_roots)
     }
 }
 
+// ---------------------------------------------------------------------------
+// root reduction of large sparse graphs
+// ---------------------------------------------------------------------------
+//
+// The leaf and triangle rules of a root (rule_leaf, rule_triangle) over a whole
+// workgroup instead of one wave, before the search: what they leave of the
+// graph becomes a graph of its own, with its vertices renumbered in their old
+// order, that the search runs on.  Bound by latency (a chain of rounds over
+// shrinking lists, a few microseconds each), so every thread works on its own
+// vertex or edge and the degrees are in LDS when they fit.  On an
+// Erdos-Renyi graph of n = 40,000 and mean degree 2 one wave took 8.3 ms for
+// these rules with its node in HBM, and every later node went on scanning
+// 40,000 vertices.
+
+// In and out of one graph (pinned host memory).
+struct ShrinkGraph {
+    uint32_t base;       // in: first word of the graph's work area
+    uint32_t n, m;       // out: what is left
+    uint32_t covered;    // out: vertices the rules put in the cover
+};
+// word offsets in a graph's work area of n vertices, m edges
+__host__ __device__ inline uint32_t shrink_ids(uint32_t) { return 0u; }                 // [n] old id of a kept vertex
+__host__ __device__ inline uint32_t shrink_cover(uint32_t n) { return n; }              // bitmap of the rules' cover
+__host__ __device__ inline uint32_t shrink_src(uint32_t n) { return n + ((n + 63u) / 64u) * 2u; }
+__host__ __device__ inline uint32_t shrink_degree(uint32_t n) { return shrink_src(n) + n + 1u; }
+__host__ __device__ inline uint32_t shrink_scratch(uint32_t n) { return shrink_degree(n) + n; }  // 7 n words
+__host__ __device__ inline uint32_t shrink_dst(uint32_t n) { return shrink_scratch(n) + 7u * n; }
+__host__ __device__ inline uint64_t shrink_words(uint32_t n, uint32_t m) { return ((uint64_t)shrink_dst(n) + 2ull * m + 15u) / 16u * 16u; }
+constexpr uint32_t kShrinkLdsMaxN = 36864;  // int32 degrees in 144 KB of LDS
+constexpr int kShrinkGone = -(1 << 30);     // degree of a vertex in the cover: negative after any number of decrements
+
+__global__ __launch_bounds__(1024) void shrink_kernel(const uint32_t *gbuf, const GDesc *gdesc, uint32_t *work,
+                                                      ShrinkGraph *graphs)
+{
+    extern __shared__ int4 smem4[];
+    __shared__ uint32_t count[4];  // next leaves, leaves' neighbours to cover, degree-2 vertices, cover size
+    __shared__ uint32_t part[2][17];
+    const uint32_t tid = threadIdx.x;
+    const GDesc &gd = gdesc[blockIdx.x];
+    const uint32_t n = gd.n;
+    const uint32_t *const src = gbuf + gd.off_src, *const dst = gbuf + gd.off_dst;
+    uint32_t *const area = work + graphs[blockIdx.x].base;
+    uint32_t *const scratch = area + shrink_scratch(n);
+    uint32_t *leaves = scratch, *next = scratch + n;
+    uint32_t *const cover = scratch + 2u * n, *const pairs = scratch + 3u * n, *const sum = scratch + 4u * n;
+    uint32_t *const marked = scratch + 5u * n;
+    int *const deg = n <= kShrinkLdsMaxN ? reinterpret_cast<int *>(smem4) : reinterpret_cast<int *>(scratch + 6u * n);
+    if (tid < 4u) count[tid] = 0u;
+    __syncthreads();
+    // degrees and sums of the live neighbours' ids (a leaf's neighbour is the sum)
+    for (uint32_t v = tid; v < n; v += 1024u) {
+        const uint32_t b = src[v], e = src[v + 1u];
+        uint32_t s = 0;
+        for (uint32_t x = b; x < e; ++x) s += dst[x];
+        deg[v] = (int)(e - b);
+        sum[v] = s;
+        marked[v] = 0u;
+        if (e - b == 1u) leaves[atomicAdd(&count[0], 1u)] = v;
+        if (e - b == 2u) pairs[atomicAdd(&count[2], 1u)] = v;
+    }
+    __syncthreads();
+    // the vertices cover[0 .. count[1]) leave the graph; new leaves and degree-2
+    // vertices are listed
+    auto apply = [&]() {
+        const uint32_t nc = count[1];
+        for (uint32_t i = tid; i < nc; i += 1024u) deg[cover[i]] = kShrinkGone;
+        __syncthreads();
+        if (tid == 0) {
+            count[0] = 0u;
+            count[3] += nc;
+        }
+        __syncthreads();
+        // eight threads per vertex
+        for (uint32_t i = tid / 8u; i < nc; i += 128u) {
+            const uint32_t u = cover[i], e = src[u + 1u];
+            for (uint32_t x = src[u] + tid % 8u; x < e; x += 8u) {
+                const uint32_t t = dst[x];
+                const int old = atomicAdd(&deg[t], -1);
+                if (old <= 0) continue;
+                atomicSub(&sum[t], u);
+                if (old == 2) next[atomicAdd(&count[0], 1u)] = t;
+                if (old == 3) pairs[atomicAdd(&count[2], 1u)] = t;
+            }
+        }
+        __syncthreads();
+        uint32_t *const x = leaves;
+        leaves = next;
+        next = x;
+    };
+    for (;;) {
+        for (;;) {
+            const uint32_t nl = count[0];
+            __syncthreads();
+            if (nl == 0u) break;
+            if (tid == 0) count[1] = 0u;
+            __syncthreads();
+            for (uint32_t i = tid; i < nl; i += 1024u) {
+                const uint32_t v = leaves[i];
+                if (ld_rlx(&deg[v]) != 1) continue;
+                const uint32_t u = ld_rlx(&sum[v]);
+                const int du = ld_rlx(&deg[u]);
+                // of an isolated edge only the lower end
+                if ((du > 1 || (du == 1 && u < v)) && atomicExch(&marked[u], 1u) == 0u) cover[atomicAdd(&count[1], 1u)] = u;
+            }
+            __syncthreads();
+            apply();
+        }
+        const uint32_t np = count[2];
+        __syncthreads();
+        if (np == 0u) break;
+        if (tid == 0) {
+            count[1] = 0u;
+            count[2] = 0u;
+        }
+        __syncthreads();
+        // the list is rewritten by apply(): read it first
+        for (uint32_t i0 = 0; i0 < np; i0 += 1024u) {
+            const uint32_t i = i0 + tid;
+            if (i >= np) continue;
+            const uint32_t v = pairs[i];
+            if (ld_rlx(&deg[v]) != 2) continue;
+            // the two live neighbours: the first by a walk, the other from the sum
+            uint32_t x = src[v];
+            while (ld_rlx(&deg[dst[x]]) < 0) ++x;
+            const uint32_t p = dst[x], q = ld_rlx(&sum[v]) - p;
+            const int dp = ld_rlx(&deg[p]), dq = ld_rlx(&deg[q]);
+            if ((dp == 2 && p < v) || (dq == 2 && q < v)) continue;  // (no degree 1 here: the leaf rule is at its end)
+            uint32_t lo = src[q], hi = src[q + 1u];
+            bool adjacent = false;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2u, y = dst[mid];
+                if (y == p) {
+                    adjacent = true;
+                    break;
+                }
+                if (y < p)
+                    lo = mid + 1u;
+                else
+                    hi = mid;
+            }
+            if (!adjacent) continue;
+            if (atomicExch(&marked[p], 1u) == 0u) cover[atomicAdd(&count[1], 1u)] = p;
+            if (atomicExch(&marked[q], 1u) == 0u) cover[atomicAdd(&count[1], 1u)] = q;
+        }
+        __syncthreads();
+        if (count[1] == 0u) break;
+        apply();
+    }
+    __syncthreads();
+    // what is left, renumbered in order: every thread counts its own run of
+    // vertices, a scan over the workgroup gives its first id and edge
+    const uint32_t per = (n + 1023u) / 1024u, v0 = min(tid * per, n), v1 = min(v0 + per, n);
+    uint32_t c = 0, de = 0;
+    for (uint32_t v = v0; v < v1; ++v) {
+        const int x = ld_rlx(&deg[v]);
+        if (x > 0) {
+            ++c;
+            de += (uint32_t)x;
+        }
+    }
+    const uint32_t ic = (uint32_t)wave_incl_scan((int)c), ie = (uint32_t)wave_incl_scan((int)de);
+    if (tid % 64u == 63u) {
+        part[0][tid / 64u] = ic;
+        part[1][tid / 64u] = ie;
+    }
+    __syncthreads();
+    if (tid < 2u) {
+        uint32_t run = 0;
+        for (uint32_t i = 0; i < 16u; ++i) {
+            const uint32_t x = part[tid][i];
+            part[tid][i] = run;
+            run += x;
+        }
+        part[tid][16] = run;
+    }
+    __syncthreads();
+    uint32_t id = part[0][tid / 64u] + ic - c, edge = part[1][tid / 64u] + ie - de;
+    uint32_t *const ids = area + shrink_ids(n), *const new_src = area + shrink_src(n), *const new_deg = area + shrink_degree(n),
+                   *const new_dst = area + shrink_dst(n), *const new_id = marked;
+    for (uint32_t v = v0; v < v1; ++v) {
+        const int x = ld_rlx(&deg[v]);
+        if (x <= 0) continue;
+        new_id[v] = id;
+        ids[id] = v;
+        new_src[id] = edge;
+        new_deg[id] = (uint32_t)x;
+        ++id;
+        edge += (uint32_t)x;
+    }
+    const uint32_t left = part[0][16], ends = part[1][16];
+    if (tid == 0) {
+        new_src[left] = ends;
+        graphs[blockIdx.x].n = left;
+        graphs[blockIdx.x].m = ends / 2u;
+        graphs[blockIdx.x].covered = count[3];
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < left; i += 1024u) {
+        const uint32_t v = ids[i];
+        uint32_t at = new_src[i];
+        for (uint32_t x = src[v]; x < src[v + 1u]; ++x) {
+            const uint32_t t = dst[x];
+            if (ld_rlx(&deg[t]) > 0) new_dst[at++] = new_id[t];
+        }
+    }
+    uint32_t *const bitmap = area + shrink_cover(n);
+    for (uint32_t base = tid / 64u * 64u; base < n; base += 1024u) {
+        const uint32_t v = base + tid % 64u;
+        const uint64_t m = __ballot(v < n && ld_rlx(&deg[v < n ? v : 0u]) < 0);
+        if (tid % 64u < 2u) bitmap[base / 32u + tid % 64u] = (uint32_t)(m >> (32u * (tid % 64u)));
+    }
+}
+
 // Read-back of vc_solve_noalloc, written inside its fixed scratch: launch
 // totals, one vc_result per graph, and every cover bitmap expanded to one
 // byte per vertex (graph g's bytes start at 32 x its first bitmap word).
@@ -2460,6 +2673,7 @@ struct vc_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;  // solve start / end / results on host
+    hipEvent_t ev_shrink = nullptr;                          // root reduction start
     int cu_count = 0;
     int wall_khz = 100000;  // device wall-clock rate
     size_t total_mem = 0;
@@ -2467,6 +2681,10 @@ struct vc_ctx {
     // launch scratch, grown on demand and reused across solves
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    // work areas and results of shrink_kernel, kept across solves
+    uint32_t *shrink_work = nullptr;
+    size_t shrink_work_words = 0;
+    vcg::ShrinkGraph *shrink_io = nullptr;  // pinned, kShrinkMaxGraphs
     // autotuner cache: (vertex-count bucket, density bucket) -> chosen params
     std::map<std::pair<int, int>, vc_params> tuned;
     // hipFree / hipHostFree wait for the whole device, including a running
@@ -2550,6 +2768,11 @@ struct DispatchKey {
 
 struct vc_graphs {
     int count = 0;
+    vc_graphs *rest = nullptr;    // what shrink_kernel leaves of the set (buffers kept across solves)
+    bool borrowed = false;        // d_words belongs to the context
+    bool dirty = false;           // h_desc differs from d_desc beyond the job fields
+    uint32_t *h_shrink = nullptr; // pinned: old ids and cover bitmaps of shrink_kernel
+    uint32_t leaf_share = 0;      // the least share of degree-1 vertices in a graph of the set, in 1/1024
     uint32_t *d_words = nullptr;  // CSR arrays of every graph
     GDesc *d_desc = nullptr;      // per-graph descriptors (job fields rewritten per solve)
     uint32_t *d_covers = nullptr; // cover bitmaps
@@ -3019,7 +3242,7 @@ vc_status vc_ctx_create(int device, vc_ctx **out)
     int khz = 0;
     if (hip_ok(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device)) && khz > 0) c->wall_khz = khz;
     if (!hip_ok(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) || !hip_ok(hipEventCreate(&c->ev0)) ||
-        !hip_ok(hipEventCreate(&c->ev1)) || !hip_ok(hipEventCreate(&c->ev2))) {
+        !hip_ok(hipEventCreate(&c->ev1)) || !hip_ok(hipEventCreate(&c->ev2)) || !hip_ok(hipEventCreate(&c->ev_shrink))) {
         delete c;
         return VC_EDEVICE;
     }
@@ -3035,11 +3258,14 @@ vc_status vc_ctx_destroy(vc_ctx *c)
     if (!c) return VC_EINVAL;
     (void)hipSetDevice(c->device);
     if (c->scratch) (void)hipFree(c->scratch);
+    if (c->shrink_work) (void)hipFree(c->shrink_work);
+    if (c->shrink_io) (void)hipHostFree(c->shrink_io);
     for (auto &x : c->deferred) free_now(x.first, x.second);
     c->deferred.clear();
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->ev2) (void)hipEventDestroy(c->ev2);
+    if (c->ev_shrink) (void)hipEventDestroy(c->ev_shrink);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return VC_OK;
@@ -3088,7 +3314,11 @@ vc_status vc_graphs_upload(vc_ctx *ctx, int count, const vc_csr *graphs, vc_grap
         }
     }
     s->cover_words = std::max<uint32_t>(cover_words, 2u);
+    s->leaf_share = 1024u;
     for (int i = 0; i < count; ++i) {
+        uint64_t leaves = 0;
+        for (uint32_t v = 0; v < graphs[i].vertexNum; ++v) leaves += graphs[i].degree[v] == 1;
+        s->leaf_share = std::min<uint32_t>(s->leaf_share, (uint32_t)(1024u * leaves / std::max<uint32_t>(1u, graphs[i].vertexNum)));
         const double n = graphs[i].vertexNum, m = graphs[i].edgeNum;
         s->mean_n += n / count;
         s->mean_density += (n > 1 ? 2.0 * m / (n * (n - 1)) : 0.0) / count;
@@ -3130,7 +3360,9 @@ vc_status vc_graphs_free(vc_ctx *ctx, vc_graphs *s)
 {
     if (!s) return VC_EINVAL;
     if (ctx) (void)hipSetDevice(ctx->device);
-    ctx_release(ctx, s->d_words, false);
+    if (s->rest) vc_graphs_free(ctx, s->rest);
+    if (!s->borrowed) ctx_release(ctx, s->d_words, false);
+    ctx_release(ctx, s->h_shrink, true);
     ctx_release(ctx, s->d_desc, false);
     ctx_release(ctx, s->d_covers, false);
     ctx_release(ctx, s->d_state, false);
@@ -3175,13 +3407,14 @@ vc_status prepare_solve(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, const v
     for (int i = 0; i < set->count; ++i) {
         const vc_job &j = jobs[i];
         if (j.instance != VC_MVC && j.instance != VC_PVC) return VC_EINVAL;
-        if (j.upper_bound > set->h_desc[i].n) return VC_EINVAL;
+        if (!set->borrowed && j.upper_bound > set->h_desc[i].n) return VC_EINVAL;
     }
     vc_status st = make_plan(ctx, set, jobs, params, pl, mem_budget);
     if (st != VC_OK) return st;
 
     // job fields of the descriptors
-    bool changed = false;
+    bool changed = set->dirty;
+    set->dirty = false;
     for (int i = 0; i < set->count; ++i) {
         GDesc &d = set->h_desc[i];
         const vc_job &j = jobs[i];
@@ -3266,11 +3499,9 @@ void fill_info(vc_launch_info *info, const vc_ctx *ctx, const Plan &pl, float ms
 
 extern "C" {
 
-vc_status vc_solve(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, const vc_params *params,
-                   vc_result *results, uint8_t *const *covers, vc_launch_info *info)
+static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, const vc_params *params, vc_result *results,
+                           uint8_t *const *covers, vc_launch_info *info)
 {
-    if (!ctx || !set_c || !jobs || !params || !results) return VC_EINVAL;
-    vc_graphs *set = const_cast<vc_graphs *>(set_c);
     Plan pl;
     vc_status st = prepare_solve(ctx, set, jobs, params, pl, 0);
     if (st != VC_OK) return st;
@@ -3409,6 +3640,193 @@ vc_status vc_solve(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, cons
     }
     fill_info(info, ctx, pl, ms, total_nodes, idle, donations, steals, hg.t0, last_exit, hg.state_bytes);
     return overall;
+}
+
+// Sets that shrink_kernel runs on: large graphs of which enough are leaves.
+// Below kShrinkMinN one wave's own root reduction in LDS is as fast as the extra
+// launch and the read-back; without leaves (a Barabasi-Albert graph of m >= 2
+// has none) the rules have little to start from and the launch is lost.
+constexpr uint32_t kShrinkMinN = 1024;
+constexpr uint32_t kShrinkMinLeaves = 64;  // of 1024
+constexpr int kShrinkMaxGraphs = 64;
+
+static bool shrinks(const vc_graphs *set, const vc_params *params)
+{
+    return set->nmax >= kShrinkMinN && set->leaf_share >= kShrinkMinLeaves && set->count <= kShrinkMaxGraphs &&
+           !(params->flags & VC_FLAG_GRAPH);
+}
+
+// vc_solve of a set that shrinks: the rules' cover first, then the search on
+// what is left (none of it: no second launch).
+static vc_status solve_shrunk(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, const vc_params *params, vc_result *results,
+                              uint8_t *const *covers, vc_launch_info *info)
+{
+    const int count = set->count;
+    for (int i = 0; i < count; ++i)
+        if (jobs[i].upper_bound > set->h_desc[i].n || (jobs[i].instance != VC_MVC && jobs[i].instance != VC_PVC)) return VC_EINVAL;
+    {
+        // refuse what the whole graphs' launch shape refuses
+        Plan pl;
+        const vc_status st = make_plan(ctx, set, jobs, params, pl);
+        if (st != VC_OK) return st;
+    }
+    constexpr unsigned kPinned = hipHostMallocCoherent | hipHostMallocMapped;
+    if (!ctx->shrink_io && !hip_ok(hipHostMalloc(reinterpret_cast<void **>(&ctx->shrink_io),
+                                                 sizeof(vcg::ShrinkGraph) * kShrinkMaxGraphs, kPinned)))
+        return VC_ENOMEM;
+    uint64_t words = 0, back = 0;  // work areas; old ids and cover bitmaps for the host
+    for (int i = 0; i < count; ++i) {
+        const GDesc &d = set->h_desc[i];
+        ctx->shrink_io[i] = vcg::ShrinkGraph{(uint32_t)words, 0u, 0u, 0u};
+        words += vcg::shrink_words(d.n, d.m);
+        back += vcg::shrink_src(d.n);
+    }
+    if (words >= 0xFFFFFFF0ull) return VC_ENOMEM;
+    if (ctx->shrink_work_words < words) {
+        ctx_release(ctx, ctx->shrink_work, false);
+        ctx->shrink_work = nullptr;
+        ctx->shrink_work_words = 0;
+        if (!hip_ok(hipMalloc(&ctx->shrink_work, words * sizeof(uint32_t)))) return VC_ENOMEM;
+        ctx->shrink_work_words = words;
+    }
+    bool want_covers = false;
+    if (covers)
+        for (int i = 0; i < count; ++i) want_covers |= covers[i] != nullptr;
+    if (want_covers && !set->h_shrink &&
+        !hip_ok(hipHostMalloc(reinterpret_cast<void **>(&set->h_shrink), back * sizeof(uint32_t), kPinned)))
+        return VC_ENOMEM;
+    const size_t smem = sizeof(int) * std::min<uint32_t>(set->nmax, vcg::kShrinkLdsMaxN);
+    hipEvent_t began = ctx->ev_shrink;
+    if (!hip_ok(hipEventRecord(began, ctx->stream))) return VC_EDEVICE;
+    hipLaunchKernelGGL(vcg::shrink_kernel, dim3(count), dim3(1024), smem, ctx->stream, set->d_words, set->d_desc,
+                       ctx->shrink_work, ctx->shrink_io);
+    if (!hip_ok(hipGetLastError())) return VC_EDEVICE;
+    if (want_covers) {
+        // ids and bitmap of a graph are its area's first words
+        uint64_t at = 0;
+        for (int i = 0; i < count; ++i) {
+            vcg::Publish pub;
+            std::memset(&pub, 0, sizeof(pub));
+            pub.src[0] = ctx->shrink_work + ctx->shrink_io[i].base;
+            pub.dst[0] = set->h_shrink + at;
+            pub.words[0] = vcg::shrink_src(set->h_desc[i].n);
+            hipLaunchKernelGGL(vcg::publish_kernel, dim3(8), dim3(256), 0, ctx->stream, pub);
+            at += pub.words[0];
+        }
+        if (!hip_ok(hipGetLastError())) return VC_EDEVICE;
+    }
+    if (!hip_ok(hipEventRecord(ctx->ev2, ctx->stream)) || !hip_ok(hipEventSynchronize(ctx->ev2))) return VC_EDEVICE;
+
+    // the set of what is left, and its jobs
+    uint32_t nmax = 0;
+    for (int i = 0; i < count; ++i) nmax = std::max(nmax, ctx->shrink_io[i].n);
+    vc_graphs *rest = set->rest;
+    std::vector<vc_job> rest_jobs(count);
+    std::vector<vc_result> rest_results(count);
+    std::vector<std::vector<uint8_t>> rest_bytes(want_covers ? count : 0);
+    std::vector<uint8_t *> rest_covers(want_covers ? count : 0, nullptr);
+    vc_status overall = VC_OK;
+    for (int i = 0; i < count; ++i) {
+        const vcg::ShrinkGraph &x = ctx->shrink_io[i];
+        vc_job &j = rest_jobs[i];
+        j = jobs[i];
+        // any valid bound is at least the rules' cover; a cover below n + 1 always exists
+        j.upper_bound = std::min(jobs[i].upper_bound - std::min(jobs[i].upper_bound, x.covered), x.n + 1u);
+        j.k = jobs[i].k - std::min(jobs[i].k, x.covered);
+    }
+    if (nmax == 0) {
+        if (info) {
+            Plan pl;
+            (void)make_plan(ctx, set, jobs, params, pl);
+            fill_info(info, ctx, pl, 0.f, (uint64_t)count, 0, 0, 0, 0, 0, 0);
+            float ms = 0.f;
+            if (hipEventElapsedTime(&ms, began, ctx->ev2) == hipSuccess) info->kernel_ms = info->active_ms = ms;
+        }
+        for (int i = 0; i < count; ++i) {
+            vc_result &r = rest_results[i];
+            std::memset(&r, 0, sizeof(r));
+            r.solved = 1u;
+            r.tree_nodes = 1u;
+            r.status = VC_OK;
+            if (jobs[i].instance == VC_MVC)
+                r.cover_from_gpu = rest_jobs[i].upper_bound > 0u;
+            else
+                r.k_found = r.cover_from_gpu = 1u;  // of size 0; k below the rules' cover: see below
+        }
+    } else {
+        if (!rest) {
+            rest = new vc_graphs();
+            rest->count = count;
+            rest->borrowed = true;
+            rest->h_desc = set->h_desc;
+            rest->cover_words = set->cover_words;
+            if (!hip_ok(hipMalloc(&rest->d_desc, sizeof(GDesc) * count)) ||
+                !hip_ok(hipMalloc(&rest->d_covers, sizeof(uint32_t) * rest->cover_words)) ||
+                !hip_ok(hipMalloc(&rest->d_state, sizeof(GState) * count))) {
+                vc_graphs_free(ctx, rest);
+                return VC_ENOMEM;
+            }
+            set->rest = rest;
+        }
+        rest->d_words = ctx->shrink_work;
+        rest->nmax = nmax;
+        rest->dirty = true;
+        for (int i = 0; i < count; ++i) {
+            const vcg::ShrinkGraph &x = ctx->shrink_io[i];
+            const uint32_t n = set->h_desc[i].n;
+            GDesc &d = rest->h_desc[i];
+            d.n = x.n;
+            d.m = x.m;
+            d.off_src = x.base + vcg::shrink_src(n);
+            d.off_dst = x.base + vcg::shrink_dst(n);
+            d.off_deg = x.base + vcg::shrink_degree(n);
+            d.off_bits = 0;
+            if (want_covers && covers[i]) {
+                rest_bytes[i].resize(std::max<uint32_t>(x.n, 1u));
+                rest_covers[i] = rest_bytes[i].data();
+            }
+        }
+        overall = solve_set(ctx, rest, rest_jobs.data(), params, rest_results.data(), want_covers ? rest_covers.data() : nullptr, info);
+        if (overall != VC_OK && overall != VC_ETIMEOUT) return overall;
+        float ms = 0.f;
+        if (info && hipEventElapsedTime(&ms, began, ctx->ev1) == hipSuccess) info->kernel_ms = ms;
+    }
+    uint64_t at = 0;
+    for (int i = 0; i < count; ++i) {
+        const vcg::ShrinkGraph &x = ctx->shrink_io[i];
+        const uint32_t n = set->h_desc[i].n;
+        vc_result &r = results[i];
+        r = rest_results[i];
+        if (jobs[i].instance == VC_MVC) {
+            r.minimum = r.cover_from_gpu ? r.minimum + x.covered : jobs[i].upper_bound;
+        } else if (jobs[i].k < x.covered) {
+            // the rules' cover alone is larger than k
+            r.k_found = r.cover_from_gpu = r.minimum = 0u;
+            r.solved = 1u;
+            r.status = VC_OK;
+        } else if (r.k_found) {
+            r.minimum += x.covered;
+        }
+        if (want_covers) {
+            const uint32_t *ids = set->h_shrink + at + vcg::shrink_ids(n), *bitmap = set->h_shrink + at + vcg::shrink_cover(n);
+            if (covers[i] && r.cover_from_gpu) {
+                for (uint32_t v = 0; v < n; ++v) covers[i][v] = (bitmap[v >> 5] >> (v & 31u)) & 1u;
+                for (uint32_t v = 0; v < x.n; ++v) covers[i][ids[v]] = rest_bytes[i][v];
+            }
+            at += vcg::shrink_src(n);
+        }
+    }
+    return overall;
+}
+
+vc_status vc_solve(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, const vc_params *params,
+                   vc_result *results, uint8_t *const *covers, vc_launch_info *info)
+{
+    if (!ctx || !set_c || !jobs || !params || !results) return VC_EINVAL;
+    vc_graphs *set = const_cast<vc_graphs *>(set_c);
+    if (!hip_ok(hipSetDevice(ctx->device))) return VC_EDEVICE;
+    return shrinks(set, params) ? solve_shrunk(ctx, set, jobs, params, results, covers, info)
+                                : solve_set(ctx, set, jobs, params, results, covers, info);
 }
 
 vc_status vc_solve_noalloc(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, const vc_params *params,
