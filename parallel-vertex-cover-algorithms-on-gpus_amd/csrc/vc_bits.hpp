@@ -49,6 +49,12 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t x)
     return (uint32_t)__builtin_amdgcn_readlane(v, 63);
 }
 
+// Word k of a mask of the first c vertices.
+__device__ __forceinline__ uint64_t low_bits(uint32_t c, uint32_t k)
+{
+    return c >= 64u * k + 64u ? ~0ull : c > 64u * k ? (1ull << (c - 64u * k)) - 1ull : 0ull;
+}
+
 template <int K>
 struct BitMask {
     uint64_t w[K];
@@ -250,6 +256,9 @@ struct BitsLds {
     {
         return reinterpret_cast<uint64_t *>(base + kCtxMask)[4u * level + k];
     }
+    // a search of a whole graph: what its first reductions put in the cover
+    // (level 0 has no parent)
+    __device__ __forceinline__ uint64_t &root_cover(uint32_t k) const { return parent_mask(0u, k); }
     __device__ __forceinline__ uint32_t &count(uint32_t level) const
     {
         return reinterpret_cast<uint32_t *>(base + kCtxMeta)[2u * level];
@@ -319,13 +328,13 @@ __device__ __forceinline__ void build_rows(const N &w, const BitsLds &lds, uint3
             x = w.off(v);
             e = w.off(v + 1u);
         }
-        // four neighbours at a time, so a lane waits once for four loads
-        for (; x < e; x += 4u) {
-            uint32_t t[4];
+        // eight neighbours in flight
+        for (; x < e; x += 8u) {
+            uint32_t t[8];
 #pragma unroll
-            for (uint32_t q = 0; q < 4u; ++q) t[q] = w.nb(min(x + q, e - 1u));
+            for (uint32_t q = 0; q < 8u; ++q) t[q] = w.nb(min(x + q, e - 1u));
 #pragma unroll
-            for (uint32_t q = 0; q < 4u; ++q) {
+            for (uint32_t q = 0; q < 8u; ++q) {
                 // a repeated last neighbour sets its bit again
                 if (w.deg(t[q]) > 0) {
                     const uint32_t p = pos[t[q]];
@@ -346,14 +355,59 @@ __device__ __forceinline__ void build_rows(const N &w, const BitsLds &lds, uint3
     w.sync();
 }
 
+// The whole graph in w (at most 64 K vertices) as the LDS context of `level`.
+template <int K, class N>
+__device__ __forceinline__ void build_whole(const N &w, const BitsLds &lds, uint32_t level)
+{
+    const uint32_t n = uni(w.n);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (64u * k >= n) break;
+        const uint32_t i = 64u * k + lane_id();
+        uint32_t r[2 * K];
+#pragma unroll
+        for (int j = 0; j < 2 * K; ++j) r[j] = 0;
+        uint32_t x = 0, e = 0;
+        if (i < n) {
+            x = w.off(i);
+            e = w.off(i + 1u);
+        }
+        // eight neighbours in flight
+        for (; x < e; x += 8u) {
+            uint32_t t[8];
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) t[q] = w.nb(min(x + q, e - 1u));
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) {
+                const uint32_t bit = 1u << (t[q] & 31u);
+#pragma unroll
+                for (int j = 0; j < 2 * K; ++j) r[j] |= (t[q] >> 5) == (uint32_t)j ? bit : 0u;
+            }
+        }
+        if (i < n) {
+            lds.id(level, i) = i;
+#pragma unroll
+            for (int j = 0; j < 2 * K; ++j) reinterpret_cast<uint32_t *>(lds.row(level, i))[j] = r[j];
+        }
+    }
+    if (lane_id() == 0) {
+        lds.count(level) = n;
+        lds.parent(level) = kNone;
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) lds.root_cover(k) = 0ull;
+    }
+    nsync<false>();
+}
+
 // Makes the context of level `to` for a node of level `from`: its nq vertices
 // with a live edge in order of increasing degree (deg: the node's degrees),
-// ties in the old order.  to == from sorts a context whose vertices are all in
-// the node.  One row (2 K readlanes) per vertex of the new context, no memory
+// ties in the old order.  `first`: the new context replaces `from` as the
+// search's first one (what the node has covered is kept in root_cover);
+// otherwise to == from sorts a context whose vertices are all in the node.  One row (2 K readlanes) per vertex of the new context, no memory
 // access but LDS.
 template <int K>
 __device__ __forceinline__ void derive(const BitsLds &lds, const BitRows<K> &rows, const BitMask<K> &live,
-                                       const uint32_t (&deg)[K], uint32_t nq, uint32_t from, uint32_t to)
+                                       const uint32_t (&deg)[K], uint32_t nq, uint32_t from, uint32_t to, bool first)
 {
     const uint32_t lane = lane_id(), slots = ctx_slots(to);
     // rank of every vertex: degree by degree, in index order
@@ -388,9 +442,11 @@ __device__ __forceinline__ void derive(const BitsLds &lds, const BitRows<K> &row
             order[rank[k]] = (uint8_t)(64u * k + lane);
             lds.id(to, rank[k]) = ids[k];
         }
-    if (to != from && lane == 0) {
+    if (lane == 0 && (first || to != from)) {
         lds.count(to) = nq;
-        lds.parent(to) = from;
+        lds.parent(to) = first ? kNone : from;
+    }
+    if (lane == 0 && !first && to != from) {
 #pragma unroll
         for (int k = 0; k < K; ++k) lds.parent_mask(to, k) = live.w[k];
     }
@@ -546,9 +602,10 @@ struct BitsWorker {
     uint32_t d;          // cover size of the node
     uint32_t level;      // its context's level
     uint32_t home;       // the published context the search started from, or kNone (the node in w)
-    uint32_t fresh;      // 1 = the context is in id order (just built)
+    uint32_t fresh;      // 1 = the first context is in id order (just built)
     uint32_t published;  // levels whose context has a valid copy in HBM, held by this search
-    uint32_t nodes, rnd; // nodes so far (for the looks), random state
+    uint32_t whole;      // 1 = the first context is the graph itself
+    uint32_t rnd;        // random state (next_random)
     uint32_t best;       // the search looks for covers smaller than this
     uint64_t live[4], settled[4];  // the node's masks (K words each)
 };
@@ -571,7 +628,7 @@ __device__ __forceinline__ void make_uniform(BitsWorker &b)
     b.home = uni(b.home);
     b.fresh = uni(b.fresh);
     b.published = uni(b.published);
-    b.nodes = uni(b.nodes);
+    b.whole = uni(b.whole);
     b.rnd = uni(b.rnd);
     b.best = uni(b.best);
 }
@@ -670,12 +727,9 @@ __device__ __forceinline__ uint32_t bit_level(const SolveArgs &a, const BitsLds 
         // the stop flag and the incumbent, and the launch's counter, are read
         // at the node's start and used at its end, so the node does not wait
         // for them
-        const bool look = (++b.nodes & a.poll_mask) == 0u;
-        unsigned long long state_next = 0, counter_next = 0;
-        if (look) {
-            state_next = ld_rlx(reinterpret_cast<unsigned long long *>(&gs->best));
-            if (a.version == 1u) counter_next = ld_rlx(&a.glob->counter);
-        }
+        const unsigned long long state_next = ld_rlx(reinterpret_cast<unsigned long long *>(&gs->best));
+        unsigned long long counter_next = 0;
+        if (a.version == 1u) counter_next = ld_rlx(&a.glob->counter);
         if (++b.pending >= b.flush_every) {
             b.total_nodes += b.pending;
             flush_nodes<STAGED>(a, gd, g, b.pending, b.moved, b.flush_every, false);
@@ -818,12 +872,19 @@ __device__ __forceinline__ uint32_t bit_level(const SolveArgs &a, const BitsLds 
                 d += 1u;
             } else {
                 const uint32_t level = ctx_level(nq);
-                const bool sort = b.fresh != 0u && level == b.level && nq == live.count() && nq == uni(lds.count(b.level));
+                const bool first = b.fresh != 0u && b.whole != 0u;
+                const bool sort = b.fresh != 0u && level == b.level &&
+                                  (first || (nq == live.count() && nq == uni(lds.count(b.level))));
                 if (level > b.level || sort) {
                     // the remainder fits a smaller context (or its context is
                     // in id order still): go on there; the node is not
                     // counted twice
-                    derive<K>(lds, rows, live, deg, nq, b.level, level);
+                    if (first && lane == 0) {
+                        const uint32_t all = lds.count(b.level);
+#pragma unroll
+                        for (int k = 0; k < K; ++k) lds.root_cover(k) = low_bits(all, k) & ~live.w[k];
+                    }
+                    derive<K>(lds, rows, live, deg, nq, b.level, level, first);
                     if ((b.published >> level) & 1u) {
                         // the copy in HBM was of the old context
                         if (lane == 0) fetch_add(ctx_users(a, b.wid * kCtxLevels + level), 0xFFFFFFFFu);
@@ -835,7 +896,7 @@ __device__ __forceinline__ uint32_t bit_level(const SolveArgs &a, const BitsLds 
                     b.fresh = 0u;
 #pragma unroll
                     for (uint32_t k = 0; k < 4u; ++k) {
-                        b.live[k] = nq >= 64u * k + 64u ? ~0ull : nq > 64u * k ? (1ull << (nq - 64u * k)) - 1ull : 0ull;
+                        b.live[k] = low_bits(nq, k);
                         b.settled[k] = 0ull;
                     }
                     return kBitsNode;
@@ -893,30 +954,29 @@ __device__ __forceinline__ uint32_t bit_level(const SolveArgs &a, const BitsLds 
                             }
                         }
                     }
-                    if (look && a.version == 1u && b.top >= b.bot && wants_donation(a, counter_next, b.rnd)) {
+                    if (a.version == 1u && b.top >= b.bot && wants_donation(a, counter_next, b.rnd)) {
                         if (uni((uint32_t)(state_next >> 32)) == 0u) return leave(kBitsDonate);
                     }
                 }
             }
         }
-        if (look) {
-            if (uni((uint32_t)(state_next >> 32))) {
-                b.top = -1;
-                b.bot = 0;
-                return kBitsDone;
-            }
-            if (mvc) b.best = min(b.best, uni((uint32_t)state_next));
+        if (uni((uint32_t)(state_next >> 32))) {
+            b.top = -1;
+            b.bot = 0;
+            return kBitsDone;
         }
+        if (mvc) b.best = min(b.best, uni((uint32_t)state_next));
     }
 }
 
 // The cover of a node of the search, one bitmap word after the other to
 // put(i, word): at its level the vertices missing from `live` (kNone: none),
 // at the levels above those missing from the mask that led down, and the cover
-// outside the first context (the home context's copy, or the node in w).
+// outside the first context (the home context's copy, root_cover, or the node
+// in w).
 // w.mark (all zero between passes) holds the search's part while it is built.
 template <class N, class F>
-__device__ __forceinline__ void cover_words(const SolveArgs &a, const N &w, const BitsLds &lds, uint32_t home, uint32_t n,
+__device__ __forceinline__ void cover_words(const SolveArgs &a, const N &w, const BitsLds &lds, uint32_t home, bool whole, uint32_t n,
                                             uint32_t level, const uint64_t *live, F &&put)
 {
     const uint32_t words = ((n + 63u) / 64u) * 2u;
@@ -942,7 +1002,10 @@ __device__ __forceinline__ void cover_words(const SolveArgs &a, const N &w, cons
         level = up;
     }
     w.sync();
-    if (home == kNone) {
+    if (whole) {
+        if (lane_id() < words)
+            put(lane_id(), (uint32_t)(lds.root_cover(lane_id() / 2u) >> (32u * (lane_id() & 1u))) | w.mark[lane_id()]);
+    } else if (home == kNone) {
         for (uint32_t base = 0; base < n; base += kWave) {
             const uint32_t v = base + lane_id();
             const uint64_t cm = __ballot(v < n && w.deg(v < n ? v : 0u) < 0);
@@ -978,7 +1041,7 @@ __device__ __forceinline__ void publish(const SolveArgs &a, const N &w, const Bi
     for (uint32_t i = lane; i < c; i += kWave)
         __builtin_amdgcn_raw_buffer_store_b32(lds.id(level, i), cb, kHbmBase + ctx_ids(level) + 4u * i, 0, kCoherent);
     if (lane == 0) __builtin_amdgcn_raw_buffer_store_b32(c, cb, kHbmCount + 4u * level, 0, kCoherent);
-    cover_words(a, w, lds, b.home, n, level, nullptr, [&](uint32_t i, uint32_t word) {
+    cover_words(a, w, lds, b.home, b.whole != 0u, n, level, nullptr, [&](uint32_t i, uint32_t word) {
         __builtin_amdgcn_raw_buffer_store_b32(word, cb, ctx_cover(a, level) + 4u * i, 0, kCoherent);
     });
     if (lane == 0) st_rlx(ctx_users(a, ctx), 1u);
@@ -991,18 +1054,25 @@ __device__ __forceinline__ void fetch_home(const SolveArgs &a, const BitsLds &ld
     const __amdgpu_buffer_rsrc_t cb = ctx_rsrc(a, b.home);
     const uint32_t cap = ctx_cap(level), row_words = cap * 2u * ctx_slots(level);
     const uint32_t c = __builtin_amdgcn_raw_buffer_load_b32(cb, kHbmCount + 4u * level, 0, kCoherent);
-    // (rows and ids past the context's vertices are read too, and not used)
-    for (uint32_t i = lane; i < row_words; i += 4u * kWave) {
-        uint32_t x[4];
+    // Eight row words and the ids in flight per lane: the round trip, some two
+    // microseconds, is what a fetch costs.  (Rows and ids past the context's
+    // vertices are read too, and not used.)
+    uint32_t id[4];
 #pragma unroll
-        for (uint32_t q = 0; q < 4u; ++q)
+    for (uint32_t q = 0; q < 4u; ++q)
+        id[q] = q * kWave < cap ? __builtin_amdgcn_raw_buffer_load_b32(cb, kHbmBase + ctx_ids(level) + 4u * (lane + q * kWave), 0, kCoherent) : 0u;
+    for (uint32_t i = lane; i < row_words; i += 8u * kWave) {
+        uint32_t x[8];
+#pragma unroll
+        for (uint32_t q = 0; q < 8u; ++q)
             x[q] = __builtin_amdgcn_raw_buffer_load_b32(cb, kHbmBase + ctx_rows(level) + 4u * (i + q * kWave), 0, kCoherent);
 #pragma unroll
-        for (uint32_t q = 0; q < 4u; ++q)
+        for (uint32_t q = 0; q < 8u; ++q)
             if (i + q * kWave < row_words) reinterpret_cast<uint32_t *>(lds.base + ctx_rows(level))[i + q * kWave] = x[q];
     }
-    for (uint32_t i = lane; i < cap; i += kWave)
-        lds.id(level, i) = __builtin_amdgcn_raw_buffer_load_b32(cb, kHbmBase + ctx_ids(level) + 4u * i, 0, kCoherent);
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q)
+        if (lane + q * kWave < cap) lds.id(level, lane + q * kWave) = id[q];
     if (lane == 0) {
         lds.count(level) = c;
         lds.parent(level) = kNone;
@@ -1031,7 +1101,6 @@ __device__ __forceinline__ void bit_search(uint64_t args, const N &w, const Bits
     b.wid = uni(b.wid);
     b.base = b.top;
     b.published = 0u;
-    b.nodes = 0u;
     b.level = 0u;
     b.fresh = 0u;
     make_uniform(b);
@@ -1042,18 +1111,27 @@ __device__ __forceinline__ void bit_search(uint64_t args, const N &w, const Bits
     if (nq != 0u) {
         b.level = ctx_level(nq);
         b.fresh = 1u;
-        if (nq <= 64u)
-            build_rows<1>(w, lds, b.level, nq);
-        else if (nq <= 128u)
-            build_rows<2>(w, lds, b.level, nq);
-        else
-            build_rows<4>(w, lds, b.level, nq);
+        if (b.whole) {
+            if (nq <= 64u)
+                build_whole<1>(w, lds, b.level);
+            else if (nq <= 128u)
+                build_whole<2>(w, lds, b.level);
+            else
+                build_whole<4>(w, lds, b.level);
+        } else {
+            if (nq <= 64u)
+                build_rows<1>(w, lds, b.level, nq);
+            else if (nq <= 128u)
+                build_rows<2>(w, lds, b.level, nq);
+            else
+                build_rows<4>(w, lds, b.level, nq);
+            b.pending -= 1u;  // the node was counted before its context was made
+        }
 #pragma unroll
         for (uint32_t k = 0; k < 4u; ++k) {
-            b.live[k] = nq >= 64u * k + 64u ? ~0ull : nq > 64u * k ? (1ull << (nq - 64u * k)) - 1ull : 0ull;
+            b.live[k] = low_bits(nq, k);
             b.settled[k] = 0ull;
         }
-        b.pending -= 1u;  // the node was counted before its context was made
     } else {
         b.level = b.home % kCtxLevels;
         fetch_home(a, lds, b);
@@ -1078,7 +1156,7 @@ __device__ __forceinline__ void bit_search(uint64_t args, const N &w, const Bits
             const uint32_t level = b.level;
             record_cover(a, gd, g, uni(b.d), [&] {
                 uint32_t *const cw = a.covers + gd.off_cover;
-                cover_words(a, w, lds, b.home, n, level, b.live, [&](uint32_t i, uint32_t x) { cw[i] = x; });
+                cover_words(a, w, lds, b.home, b.whole != 0u, n, level, b.live, [&](uint32_t i, uint32_t x) { cw[i] = x; });
             });
             if (uni(gd.instance) == 0u) b.best = min(b.best, b.d);
             pop = true;

@@ -59,13 +59,15 @@ struct Global {
     // updated with single 64-bit atomics so a dequeue moves a worker out of
     // "waiting" and an item out of "enqueued" in one step (the reference packs
     // {numWaiting, numEnqueued} the same way, src/BWDWorkList.cuh:8-11,200-205).
+    // "enqueued" is signed: workers that find nothing there take it below 0
+    // for a moment.
     unsigned long long counter;
     uint32_t pad0[14];
     unsigned long long head;  // 64-bit ring positions (the reference uses two
     uint32_t pad1[14];        // 32-bit halves of one word, src/BWDWorkList.cuh:63-69)
     unsigned long long tail;
     uint32_t pad2[14];
-    int32_t count;            // occupancy guard (src/BWDWorkList.cuh:78-110)
+    int32_t count;            // occupancy guard of small rings (src/BWDWorkList.cuh:78-110)
     uint32_t pad3[15];
     uint32_t next_root;       // root / static-path hand-out counter
     uint32_t pad4[15];
@@ -152,6 +154,7 @@ struct SolveArgs {
     uint32_t depth;         // stack slots per worker
     uint32_t qsize;         // power of two
     uint32_t qthreshold;    // donate while enqueued < qthreshold
+    uint32_t ring_guard;    // 1 = the ring can fill (fewer than two slots per worker)
     uint32_t workers;
     uint32_t version;       // 0 static split (stack only), 1 hybrid
     uint32_t start_depth;   // static split depth
@@ -182,10 +185,6 @@ struct SolveArgs {
     // nearly all busy (0 = every worker starts at once)
     uint32_t active0;
     uint64_t dormant_ticks;
-    // bitset searches look at the graph's and the launch's shared words at
-    // every node (0) or every poll_mask + 1 nodes: with thousands of workers
-    // these reads contend on a handful of lines
-    uint32_t poll_mask;
     // node-budget flushes: workers per graph, the least number of workers
     // assumed to share a graph (vcg::flush_interval)
     uint32_t flush_share;

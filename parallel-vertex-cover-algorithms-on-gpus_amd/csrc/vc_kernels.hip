@@ -1051,11 +1051,19 @@ __device__ __forceinline__ void init_root(const N &w, const int32_t *deg0, uint3
         int dv = -1;
         if (v < w.n) {
             dv = deg0[v];
+            // eight neighbours in flight: a lane that waits for each one takes
+            // a memory round trip per neighbour
             const uint32_t e = w.off(v + 1);
-            for (uint32_t x = w.off(v); x < e; ++x) {
-                const uint32_t u = w.nb(x);
-                s += u;
-                q += (S2)u * (S2)u;
+            for (uint32_t x = w.off(v); x < e; x += 8u) {
+                uint32_t u[8];
+#pragma unroll
+                for (uint32_t j = 0; j < 8u; ++j) u[j] = w.nb(min(x + j, e - 1u));
+#pragma unroll
+                for (uint32_t j = 0; j < 8u; ++j) {
+                    const uint32_t t = x + j < e ? u[j] : 0u;
+                    s += t;
+                    q += (S2)t * (S2)t;
+                }
             }
         }
         w.init_vertex(v, dv, s, q);
@@ -1238,18 +1246,21 @@ __device__ __forceinline__ uint32_t copy_bytes(uint32_t cnt)
 // broker worklist (src/BWDWorkList.cuh) with 64-bit ring positions
 // ---------------------------------------------------------------------------
 
-// Reserves a ring slot if the occupancy guard admits one more item (the
-// caller has already decided that a donation is wanted), and counts the
-// donated subtree as one more outstanding unit of graph g.  The caller then
-// writes the slot's data and its (g, d, v, kind) with agent-coherent stores and
-// calls publish_slot.
+// Reserves a ring slot (the caller has already decided that a donation is
+// wanted), and counts the donated subtree as one more outstanding unit of
+// graph g.  The caller then writes the slot's data and its (g, d, v, kind) with
+// agent-coherent stores and calls publish_slot.  A ring of at least two slots
+// per worker cannot fill: donations stop at as many items as workers wait, and
+// every worker can be one item ahead of what it saw.  Smaller rings (-q) go
+// through the occupancy guard, which costs one more round trip.
 __device__ __forceinline__ bool reserve_slot(const SolveArgs &a, uint32_t g, uint32_t &slot_out, uint32_t &ticket_out)
 {
-    uint32_t ok = 0, slot = 0, ticket = 0;
+    uint32_t ok = 1, slot = 0, ticket = 0;
     if (lane_id() == 0) {
-        int c = fetch_add(&a.glob->count, 1);
-        if (c < (int)a.qsize) {
-            ok = 1;
+        if (a.ring_guard && fetch_add(&a.glob->count, 1) >= (int)a.qsize) {
+            fetch_add(&a.glob->count, -1);
+            ok = 0;
+        } else {
             unsigned long long pos = fetch_add(&a.glob->tail, 1ull);
             slot = (uint32_t)(pos & (unsigned long long)(a.qsize - 1));
             ticket = (uint32_t)(2ull * (pos / a.qsize));
@@ -1265,8 +1276,6 @@ __device__ __forceinline__ bool reserve_slot(const SolveArgs &a, uint32_t g, uin
             }
             // the subtree being donated is one more outstanding unit of g
             if (ok) fetch_add(&a.gstate[g].outstanding, 1u);
-        } else {
-            fetch_add(&a.glob->count, -1);
         }
     }
     ok = uni(ok);
@@ -1332,7 +1341,7 @@ __device__ __forceinline__ uint32_t next_random(uint32_t &state)
 // took 48 ms, against 17 ms on 1,024 workers.
 __device__ __forceinline__ bool wants_donation(const SolveArgs &a, unsigned long long counter, uint32_t &rnd)
 {
-    const uint32_t lo = uni((uint32_t)counter), enq = uni((uint32_t)(counter >> 32));
+    const uint32_t lo = uni((uint32_t)counter), enq = (uint32_t)max((int)uni((uint32_t)(counter >> 32)), 0);
     const uint32_t waiting = lo & 0xFFFFu, busy = (lo >> 16) - waiting;
     if (waiting == 0u || enq >= waiting || enq >= a.qthreshold) return false;
     const uint32_t missing = waiting - enq;
@@ -1340,33 +1349,29 @@ __device__ __forceinline__ bool wants_donation(const SolveArgs &a, unsigned long
     return ((next_random(rnd) * busy) >> 16) < 2u * missing;
 }
 
-// Takes one item if the occupancy guard says one is there.  On success
+// Takes the next item of the ring; the caller has taken one off the
+// "enqueued" field, so there is one.  On success
 // (g, d, v) are returned and either the node state is in the worker's node
 // storage (ctx = kNone), or the item is a subtree of the bitset search of
-// context ctx: word i < v of its masks in lane i of `word`.
+// context ctx: word i < v of its masks in lane i of `word`.  False when the
+// launch is being cancelled.
 template <bool SERVE, class N>
-__device__ bool try_dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_t &d, uint32_t &v, uint32_t &ctx,
-                            uint32_t &word, uint32_t slot_bytes)
+__device__ __forceinline__ bool dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_t &d, uint32_t &v, uint32_t &ctx,
+                                        uint32_t &word, uint32_t slot_bytes)
 {
-    uint32_t ok = 0, slot = 0, ticket = 0;
-    if (lane_id() == 0 && ld_rlx(&a.glob->count) > 0) {
-        int c = fetch_add(&a.glob->count, -1);
-        if (c > 0) {
-            ok = 1;
-            unsigned long long pos = fetch_add(&a.glob->head, 1ull);
-            slot = (uint32_t)(pos & (unsigned long long)(a.qsize - 1));
-            ticket = (uint32_t)(2ull * (pos / a.qsize) + 1ull);
-            uint32_t spins = 0;
-            while (ld_rlx(&a.tickets[slot]) != ticket) {
-                backoff(spins < 3 ? spins : 3);
-                ++spins;
-                if (past_deadline(a)) {
-                    ok = 0;  // the launch is being cancelled: leave the slot alone
-                    break;
-                }
+    uint32_t ok = 1, slot = 0, ticket = 0;
+    if (lane_id() == 0) {
+        unsigned long long pos = fetch_add(&a.glob->head, 1ull);
+        slot = (uint32_t)(pos & (unsigned long long)(a.qsize - 1));
+        ticket = (uint32_t)(2ull * (pos / a.qsize) + 1ull);
+        uint32_t spins = 0;
+        while (ld_rlx(&a.tickets[slot]) != ticket) {
+            backoff(spins < 3 ? spins : 3);
+            ++spins;
+            if (past_deadline(a)) {
+                ok = 0;  // the launch is being cancelled: leave the slot alone
+                break;
             }
-        } else {
-            fetch_add(&a.glob->count, 1);
         }
     }
     ok = uni(ok);
@@ -1381,16 +1386,17 @@ __device__ bool try_dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_
     else
         handoff_observe();
     const u32x4 m = __builtin_amdgcn_raw_buffer_load_b128(slot_rsrc(&a.q_meta[slot], 16u), 0u, 0, kCoherent);
+    // the masks of a bitset subtree, in flight with its descriptor
+    word = 0;
+    if (lane_id() < 16u)
+        word = __builtin_amdgcn_raw_buffer_load_b32(
+            slot_rsrc(static_cast<const char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes), 4u * lane_id(), 0, kCoherent);
     g = uni(m.x);
     d = uni(m.y);
     v = uni(m.z);
     ctx = uni(m.w) - 1u;
-    word = 0;
     if (ctx != kNone) {
-        if (lane_id() < v)
-            word = __builtin_amdgcn_raw_buffer_load_b32(
-                slot_rsrc(static_cast<const char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes), 4u * lane_id(), 0,
-                kCoherent);
+        // nothing else to copy
     } else if constexpr (N::kPacked && !N::kHbm)
         copy_state_to_lds<N, true>(w.base, static_cast<const char *>(a.q_deg) + (size_t)slot * slot_bytes, a.npad,
                                    uni(a.gdesc[g].n));
@@ -1401,8 +1407,7 @@ __device__ bool try_dequeue(const SolveArgs &a, const N &w, uint32_t &g, uint32_
     handoff_publish();  // the slot's loads are complete before it is freed
     if (lane_id() == 0) {
         st_rlx(&a.tickets[slot], ticket + 1u);
-        // leave "waiting" and take the item off "enqueued" in one step
-        fetch_add(&a.glob->counter, (unsigned long long)(0ull - (kEnqOne + kWaitOne)));
+        if (a.ring_guard) fetch_add(&a.glob->count, -1);
     }
     return true;
 }
@@ -1661,16 +1666,10 @@ struct Acquired {
 // registers as registered-and-waiting in one atomic at its start).
 //
 // Batch launches count their roots in the termination word's "enqueued"
-// field from the start (init_kernel), like items of the worklist: a claim
-// takes the root index from next_root and then leaves "waiting" and
-// "enqueued" in one atomic, so termination is simply waiting == registered
-// with nothing enqueued, and a failed claim undoes nothing.  At a worker's
-// start only the first `roots` workers to register try to claim roots (the
-// others join in after two polls): with one root and 7,168 workers every
-// worker's claim attempt on the same words cost more than the search of a
-// small graph.
+// field from the start (init_kernel), like items of the worklist, so
+// termination is simply waiting == registered with nothing enqueued.
 template <bool SERVE, class N>
-__device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes, bool counted, uint32_t rid, uint32_t rnd)
+__device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes, bool counted, uint32_t rnd)
 {
     Acquired r = {0u, kNone, 0u, kNone, 0u, kNone, 0u};
     // A cancelled or late launch hands out no more work.  Checked on every
@@ -1690,10 +1689,32 @@ __device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes,
         const unsigned long long seen = ld_rlx(&a.glob->counter);
         const uint32_t lo = uni((uint32_t)seen), hi = uni((uint32_t)(seen >> 32));
         const uint32_t waiting = lo & 0xFFFFu, reg = lo >> 16;
-        const bool attempt = hi != 0u && (2u * hi >= waiting || ((next_random(rnd) * waiting) >> 16) < 2u * hi);
-        if (a.version == 1 && attempt) {
-            uint32_t g, d, v, ctx, word;
-            if (try_dequeue<SERVE>(a, w, g, d, v, ctx, word, slot_bytes)) {
+        if ((int)hi > 0 && (2u * hi >= waiting || ((next_random(rnd) * waiting) >> 16) < 2u * hi)) {
+            // Take one off "enqueued" and leave "waiting" in one step; with
+            // nothing there (the field was 0 or, while others are at this
+            // point, below) put both back.  What was taken stands for
+            // a root while there are any, then for an item of the ring.
+            uint32_t got = 0;
+            if (lane_id() == 0) {
+                const unsigned long long old = fetch_add(&a.glob->counter, (unsigned long long)(0ull - (kEnqOne + kWaitOne)));
+                got = (int)(uint32_t)(old >> 32) > 0;
+                if (!got) fetch_add(&a.glob->counter, kEnqOne + kWaitOne);
+            }
+            if (uni(got)) {
+                if constexpr (!SERVE) {
+                    uint32_t idx = kNone;
+                    if (uni(ld_rlx(&a.glob->next_root)) < a.roots) {
+                        if (lane_id() == 0) idx = fetch_add(&a.glob->next_root, 1u);
+                        idx = uni(idx);
+                    }
+                    if (idx < a.roots) {
+                        r.kind = 2;
+                        r.root = idx;
+                        return r;
+                    }
+                }
+                uint32_t g, d, v, ctx, word;
+                if (!dequeue<SERVE>(a, w, g, d, v, ctx, word, slot_bytes)) return r;  // cancelled
                 r.kind = 1;
                 r.g = g;
                 r.d = d;
@@ -1703,21 +1724,7 @@ __device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes,
                 return r;
             }
         }
-        if constexpr (!SERVE) {
-            if (hi != 0u && (rid < a.roots || spins >= 2u) && uni(ld_rlx(&a.glob->next_root)) < a.roots) {
-                uint32_t idx = kNone;
-                if (lane_id() == 0) {
-                    idx = fetch_add(&a.glob->next_root, 1u);
-                    if (idx < a.roots) fetch_add(&a.glob->counter, (unsigned long long)(0ull - (kEnqOne + kWaitOne)));
-                }
-                idx = uni(idx);
-                if (idx < a.roots) {
-                    r.kind = 2;
-                    r.root = idx;
-                    return r;
-                }
-            }
-        } else {
+        if constexpr (SERVE) {
             const uint32_t avail = roots_available<SERVE>(a);
             if (uni(ld_rlx(&a.glob->next_root)) < avail) {
                 uint32_t idx = kNone;
@@ -1795,7 +1802,7 @@ __device__ bool dormant_join(const SolveArgs &a, uint32_t wid)
     uint64_t interval = a.dormant_ticks;
     uint32_t h = wid * 2654435761u;
     uint64_t next = start + (interval * (128u + (h >> 24))) / 256u;
-    const uint64_t quantum = a.dormant_ticks / 4u;
+    const uint64_t quantum = a.dormant_ticks / 16u;
     uint64_t look = start + quantum;
     for (;;) {
         for (;;) {
@@ -1808,7 +1815,7 @@ __device__ bool dormant_join(const SolveArgs &a, uint32_t wid)
                 h = h * 1664525u + 1013904223u;
                 look = now + (quantum * (128u + (h >> 24))) / 256u;
             }
-            __builtin_amdgcn_s_sleep(127);
+            __builtin_amdgcn_s_sleep(32);
         }
         unsigned long long c = 0;
         uint32_t over = 0;
@@ -1817,7 +1824,7 @@ __device__ bool dormant_join(const SolveArgs &a, uint32_t wid)
             over = ld_rlx(&a.glob->done_flag) | ld_rlx(&a.glob->cancel);
         }
         if (uni(over)) return false;
-        const uint32_t lo = uni((uint32_t)c), enq = uni((uint32_t)(c >> 32));
+        const uint32_t lo = uni((uint32_t)c), enq = (uint32_t)max((int)uni((uint32_t)(c >> 32)), 0);
         const uint32_t waiting = lo & 0xFFFFu, reg = lo >> 16;
         const uint64_t now = wall_clock64();
         const uint64_t elapsed = now - start;
@@ -1892,8 +1899,20 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     const uint32_t wib = threadIdx.x / kWave;
     const uint32_t wid = blockIdx.x * (blockDim.x / kWave) + wib;
     if (wid >= a.workers) return;
-    if constexpr (STAGED)
-        if (wid >= a.active0 && !dormant_join(a, wid)) return;
+    if constexpr (STAGED) {
+        // (active0 is a multiple of the workers per workgroup)
+        if (wid >= a.active0) {
+            uint32_t *const join = reinterpret_cast<uint32_t *>(smem4);
+            if (wib == 0u) {
+                const bool yes = dormant_join(a, wid);
+                if (lane_id() == 0) *join = yes;
+            }
+            __syncthreads();
+            const uint32_t yes = *join;
+            __syncthreads();
+            if (!uni(yes)) return;
+        }
+    }
 
     // LDS: the contexts of every worker's bitset searches, then (LDS variants)
     // the node storage
@@ -1938,11 +1957,9 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     char *stk = static_cast<char *>(a.stk) + (size_t)wid * a.depth * slot_bytes;
     uint2 *stk_meta = a.stk_meta + (size_t)wid * a.depth;
 
-    // register as a worker that waits for work, in one atomic; rid = the
-    // number of workers registered before this one
-    uint32_t rid = 0;
+    // register as a worker that waits for work, in one atomic
     if (lane_id() == 0) {
-        rid = (uint32_t)(fetch_add(&a.glob->counter, kRegOne + kWaitOne) >> 16) & 0xFFFFu;
+        fetch_add(&a.glob->counter, kRegOne + kWaitOne);
         // the time limit counts from the first worker's start, not from the
         // launch: a persistent kernel can wait for CUs held by another one
         uint64_t zero = 0;
@@ -1950,7 +1967,6 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
             __hip_atomic_compare_exchange_strong(&a.glob->t0, &zero, (uint64_t)wall_clock64(),
                                                  __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    rid = uni(rid);
     bool counted = true;  // the first acquire: already counted as waiting
 
     uint32_t g = kNone;
@@ -1970,8 +1986,10 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     uint32_t rnd = wid * 2654435761u;    // random state (next_random)
 
     for (;;) {
-        // a subtree for the bitset search: its live vertices, or a donated one
+        // a subtree for the bitset search: its live vertices (whole: a root's
+        // graph as it is), or a donated one
         uint32_t bits = 0, bits_ctx = kNone, bits_word = 0;
+        bool whole = false;
         if (!have) {
             if (top < bot) {
                 top = -1;
@@ -2003,7 +2021,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 }
                 if (lane_id() == 0 && ld_rlx(&a.glob->cancel)) st_rlx(&a.glob->done_flag, 1u);
                 const uint64_t t_idle = wall_clock64();
-                Acquired q = acquire<SERVE>(a, w, slot_bytes, counted, rid, rnd ^ (uint32_t)t_idle);
+                Acquired q = acquire<SERVE>(a, w, slot_bytes, counted, rnd ^ (uint32_t)t_idle);
                 counted = false;
                 idle_ticks += wall_clock64() - t_idle;
                 if (q.kind == 0) break;
@@ -2048,6 +2066,13 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     cands_reset(c, q.v == kNone);
                     if (q.v != kNone) d += take_neighbours(w, q.v, c);
                     descend = 0;
+                } else if (a.version == 1 && w.n - 1u < a.bits_max) {
+                    // a small graph needs no node state: its rows straight
+                    // from the adjacency, its first reductions on masks
+                    d = 0;
+                    descend = 0;
+                    bits = w.n;
+                    whole = true;
                 } else {
                     init_root(w, reinterpret_cast<const int32_t *>(a.gbuf + gd.off_deg), a.npad);
                     cands_reset(c, true);
@@ -2065,7 +2090,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
 
         GState *const gs = &a.gstate[g];
         uint32_t v = kNone;
-        if (bits_ctx == kNone) {
+        if (bits == 0u && bits_ctx == kNone) {
             // the stop flag and the incumbent in flight together (one round
             // trip to L2 per node instead of two)
             const unsigned long long state_now = ld_rlx(reinterpret_cast<unsigned long long *>(&gs->best));
@@ -2151,6 +2176,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
             bw.flush_every = flush_every;
             bw.d = d;
             bw.home = bits_ctx;
+            bw.whole = whole;
             bw.rnd = rnd;
             const uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();  // a
             bit_search<STAGED>(args, w, bits_lds, gd, g, bits, bits_word, bw);
@@ -3135,6 +3161,7 @@ void fill_args(SolveArgs &a, const Plan &pl, char *base, uint32_t version, uint3
     a.depth = pl.depth;
     a.qsize = pl.qsize;
     a.qthreshold = pl.qthreshold;
+    a.ring_guard = pl.qsize < 2u * pl.workers;
     a.workers = pl.workers;
     a.version = version;
     a.start_depth = version == VC_STACK_ONLY ? start_depth : 0u;
@@ -3457,13 +3484,12 @@ SolveArgs solve_args(const vc_ctx *ctx, const vc_graphs *set, const vc_params *p
     // deadline on the device wall clock (every wait loop checks it)
     const uint64_t ms = params->time_limit_ms ? params->time_limit_ms : 3600ull * 1000ull;
     fill_args(a, pl, base, params->version, params->start_depth, ms * (uint64_t)ctx->wall_khz);
-    a.poll_mask = 0u;
     a.flush_share = std::max<uint32_t>(1u, pl.workers / std::max<uint32_t>(1u, a.num_graphs));
     // staged start (vcg::dormant_join) when the grid is automatic and the
     // roots could keep fewer than half the workers busy; the adjacency
     // kernel is always staged (active0 >= workers: every worker starts)
     if (pl.adj || (!params->num_blocks && 2ull * pl.roots < pl.workers && kActiveStart < pl.workers)) {
-        a.active0 = std::max<uint32_t>(kActiveStart, 2u * pl.roots);
+        a.active0 = round_up(std::max<uint32_t>(kActiveStart, 2u * pl.roots), pl.wpb);
         a.dormant_ticks = (uint64_t)ctx->wall_khz / 10u;  // 100 us
     }
     return a;
