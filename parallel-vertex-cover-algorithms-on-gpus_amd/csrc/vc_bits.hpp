@@ -205,12 +205,12 @@ __device__ __forceinline__ uint32_t ctx_level(uint32_t c)
 __device__ __forceinline__ uint32_t ctx_slots(uint32_t level) { return level == 0u ? 4u : level < 3u ? 2u : 1u; }
 // LDS per worker: rows of levels 1 to 5 (8 K bytes per vertex) | their ids
 // (4 bytes each) | per level a parent mask (32 bytes) | per level (vertices,
-// parent level) | 256 bytes of order scratch | rows of level 0 | its ids.
+// parent level) | 512 bytes of scratch | rows of level 0 | its ids.
 // The part before level 0 is what a worker needs with kBitsMaxSmall.  A load
 // of 64 K rows may run past its level's rows, into the next level's or the ids;
 // those lanes' vertices are in no mask.
 constexpr uint32_t kCtxIds = 4736, kCtxMask = kCtxIds + 4u * 368u, kCtxMeta = kCtxMask + 32u * kCtxLevels,
-                   kCtxOrder = kCtxMeta + 8u * kCtxLevels, kCtxRows0 = kCtxOrder + 256u, kCtxIds0 = kCtxRows0 + 8192u,
+                   kCtxOrder = kCtxMeta + 8u * kCtxLevels, kCtxRows0 = kCtxOrder + 512u, kCtxIds0 = kCtxRows0 + 8192u,
                    kCtxLdsSmall = kCtxRows0, kCtxLdsBytes = kCtxIds0 + 1024u;
 static_assert(kCtxLdsBytes % 16u == 0u && kCtxLdsSmall % 16u == 0u, "the node storage after it is 16-byte aligned");
 __device__ __forceinline__ uint32_t ctx_rows(uint32_t level)
@@ -267,7 +267,9 @@ struct BitsLds {
     {
         return reinterpret_cast<uint32_t *>(base + kCtxMeta)[2u * level + 1u];
     }
+    // scratch, a byte per vertex each
     __device__ __forceinline__ uint8_t *order() const { return reinterpret_cast<uint8_t *>(base + kCtxOrder); }
+    __device__ __forceinline__ uint8_t *claim() const { return reinterpret_cast<uint8_t *>(base + kCtxOrder + 256u); }
 };
 
 template <int K>
@@ -478,13 +480,23 @@ __device__ __forceinline__ void derive(const BitsLds &lds, const BitRows<K> &row
     nsync<false>();
 }
 
-// Greedy clique cover of the nq vertices in q: each clique starts at the first
-// unassigned vertex and takes the first common neighbour of its members
-// until none is left.  A clique of s vertices needs s - 1 of them in any
-// cover, so the cover grows by at least lb = nq - cliques.  Ends early
-// (returns true) once lb > room, the most vertices the cover may still take.
-// One vertex costs a row (2 K readlanes) and some 20 scalar instructions, no
-// memory access.
+// Greedy clique cover of the nq vertices in q.  A clique of s vertices needs
+// s - 1 of them in any cover, so the cover grows by at least lb = nq - cliques.
+// Ends early (returns true) once lb > room, the most vertices the cover may
+// still take.
+//
+// In order of the vertices: each clique starts at the first unassigned vertex
+// and takes the first common neighbour of its members until none is left.
+// That is one vertex after the other, some 200 cycles each (a row by
+// readlanes, then scalar instructions, no memory access).  In a sparse
+// remainder most of it is done by kRounds rounds for all lanes at once first:
+// vertices that are each other's first unassigned neighbour become a pair, and
+// each pair takes its first unassigned common neighbour (of several pairs that
+// want the same vertex one gets it).  Three rounds leave 14-23% of a sparse
+// remainder for the serial part and the searches visit as many nodes as
+// without them; dense remainders, whose cliques are larger, take the serial
+// part alone (with rounds the searches visit a fifth more nodes at half of all
+// edges).
 //
 // When lb <= room: any cover of at most `room` more vertices leaves at least
 // nq - room vertices out, no two in one clique, and nq - lb - r cliques with
@@ -493,6 +505,8 @@ __device__ __forceinline__ void derive(const BitsLds &lds, const BitRows<K> &row
 // cliques, singletons first, then pairs, when these are at most kFewBranch
 // vertices, and is left empty otherwise.  One such vertex: it stays out, its
 // neighbours are in, nothing is left to branch on.
+constexpr uint32_t kRounds = 3;
+constexpr uint32_t kSerialOnly = 16;  // a rest this small is left to the serial part
 constexpr uint32_t kFewBranch = 4;
 
 // The first vertex of p (not empty): off q, and p keeps its neighbours.  One
@@ -533,16 +547,90 @@ __device__ __forceinline__ uint32_t take_first(const BitRows<K> &rows, BitMask<K
 }
 
 template <int K>
-__device__ __forceinline__ bool clique_cover(const BitRows<K> &rows, BitMask<K> q, uint32_t nq, uint32_t room,
-                                             BitMask<K> &branch, uint32_t &nbranch)
+__device__ __forceinline__ bool clique_cover(const BitsLds &lds, const char *my_rows, const BitRows<K> &rows, BitMask<K> q,
+                                             uint32_t nq, uint32_t room, bool sparse, BitMask<K> &branch, uint32_t &nbranch)
 {
-    BitMask<K> one, pair_a, pair_b;  // singletons, the last two pairs
+    const uint32_t lane = lane_id();
+    BitMask<K> one, pair_a, pair_b;  // singletons, the serial part's last two pairs
+    BitMask<K> leads;                // first vertices of the rounds' pairs
+    uint32_t mate[K];                // of those
     one.clear();
     pair_a.clear();
     pair_b.clear();
+    leads.clear();
     uint32_t lb = 0, left = nq, pairs = 0;
     branch.clear();
     nbranch = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) mate[k] = 0;
+    if (sparse) {
+        uint8_t *const wants = lds.order(), *const claim = lds.claim();
+        for (uint32_t round = 0; round < kRounds && left > kSerialOnly; ++round) {
+            if (lb + left + kFewBranch <= room) return false;
+            uint32_t first[K], third[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const uint32_t v = 64u * k + lane;
+                uint32_t p = kNone;
+#pragma unroll
+                for (int j = 2 * K - 1; j >= 0; --j) {
+                    const uint32_t x = rows.r[k][j] & q.half(j);
+                    if (x) p = 32u * j + (uint32_t)__builtin_ctz(x);
+                }
+                first[k] = lane_in(q.w[k]) ? p : kNone;
+                if (lane_in(q.w[k])) {
+                    wants[v] = (uint8_t)(p != kNone ? p : v);
+                    claim[v] = 255u;  // (no pair's first vertex)
+                }
+            }
+            nsync<false>();
+            BitMask<K> paired, lead;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const uint32_t v = 64u * k + lane, p = first[k];
+                const bool mutual = (p != kNone) & (wants[p != kNone ? p : 0u] == v);
+                paired.w[k] = __ballot(mutual);
+                lead.w[k] = __ballot(mutual & (v < p));
+            }
+            if (!paired.any()) break;
+            q.drop(paired);
+            const uint32_t made = lead.count();
+            left -= 2u * made;
+            lb += made;
+            // each pair's first unassigned common neighbour
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                third[k] = kNone;
+                const uint32_t p = lane_in(lead.w[k]) ? first[k] : 0u;
+                const uint32_t *const other = reinterpret_cast<const uint32_t *>(my_rows + p * (8u * K));
+#pragma unroll
+                for (int j = 2 * K - 1; j >= 0; --j) {
+                    const uint32_t x = rows.r[k][j] & other[j] & q.half(j);
+                    if (x) third[k] = 32u * j + (uint32_t)__builtin_ctz(x);
+                }
+                if (!lane_in(lead.w[k])) third[k] = kNone;
+                if (third[k] != kNone) claim[third[k]] = (uint8_t)(64u * k + lane);
+            }
+            nsync<false>();
+            BitMask<K> joined;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const uint32_t v = 64u * k + lane;
+                joined.w[k] = __ballot(claim[v] != 255u) & q.w[k];
+                const bool got = (third[k] != kNone) & (claim[third[k] != kNone ? third[k] : 0u] == v);
+                const uint64_t alone = lead.w[k] & ~__ballot(got);
+                leads.w[k] |= alone;
+                if (lane_in(alone)) mate[k] = first[k];
+            }
+            nsync<false>();
+            q.drop(joined);
+            const uint32_t more = joined.count();
+            left -= more;
+            lb += more;
+            if (lb > room) return true;
+        }
+        pairs = leads.count();
+    }
     while (left) {
         // even one clique of all that is left leaves more than kFewBranch
         // cliques to branch in
@@ -582,8 +670,25 @@ __device__ __forceinline__ bool clique_cover(const BitRows<K> &rows, BitMask<K> 
         const uint32_t two = r - singles;
         if (two > pairs || two > 2u || singles + 2u * two > kFewBranch) return false;
         branch = one;
-        branch.add(pair_a);
-        if (two == 2u) branch.add(pair_b);
+        for (uint32_t i = 0; i < two; ++i) {
+            // the serial part's pairs first, then the rounds'
+            if (i == 0u && pair_a.any()) {
+                branch.add(pair_a);
+            } else if (i == 1u && pair_b.any()) {
+                branch.add(pair_b);
+            } else {
+                const uint32_t v = leads.last();
+                leads.reset(v);
+                uint32_t u = 0;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const uint32_t mate_k = (uint32_t)__builtin_amdgcn_readlane((int)mate[k], (int)(v & 63u));
+                    u = v / 64u == (uint32_t)k ? mate_k : u;
+                }
+                branch.set(v);
+                branch.set(u);
+            }
+        }
         nbranch = singles + 2u * two;
     }
     return false;
@@ -901,7 +1006,7 @@ __device__ __forceinline__ uint32_t bit_level(const SolveArgs &a, const BitsLds 
                     }
                     return kBitsNode;
                 }
-                dead = clique_cover<K>(rows, q, nq, room, branch, nbranch);
+                dead = clique_cover<K>(lds, my_rows, rows, q, nq, room, 4u * e2 <= nq * nq, branch, nbranch);
                 if (!dead) {
                     // children: stack all but the last
                     auto push = [&](const BitMask<K> &m, uint32_t dm) {
