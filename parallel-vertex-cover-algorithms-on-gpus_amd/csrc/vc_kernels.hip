@@ -1249,9 +1249,9 @@ __device__ __forceinline__ uint32_t copy_bytes(uint32_t cnt)
 // Reserves a ring slot (the caller has already decided that a donation is
 // wanted), and counts the donated subtree as one more outstanding unit of
 // graph g.  The caller then writes the slot's data and its (g, d, v, kind) with
-// agent-coherent stores and calls publish_slot.  A ring of at least two slots
+// agent-coherent stores and calls publish_slot.  A ring of at least six slots
 // per worker cannot fill: donations stop at as many items as workers wait, and
-// every worker can be one item ahead of what it saw.  Smaller rings (-q) go
+// every worker can be kDonateBatch items ahead of what it saw.  Smaller rings (-q) go
 // through the occupancy guard, which costs one more round trip.
 __device__ __forceinline__ bool reserve_slot(const SolveArgs &a, uint32_t g, uint32_t &slot_out, uint32_t &ticket_out)
 {
@@ -1311,17 +1311,60 @@ __device__ bool try_enqueue(const SolveArgs &a, const N &w, const char *src, uin
     return true;
 }
 
-// The same for a subtree of the bitset search (vc_bits.hpp) at context `ctx`:
-// word i < words of its masks in lane i.
-__device__ __forceinline__ bool try_enqueue_bits(const SolveArgs &a, uint32_t g, uint32_t d, uint32_t ctx, uint32_t words,
-                                                 uint32_t word, uint32_t slot_bytes)
+// The same for up to kDonateBatch subtrees of the bitset search (vc_bits.hpp) at
+// context `ctx`: the stack entries bot .. bot + count - 1, sixteen lanes and
+// words each.  A donation is a chain of four round trips to memory shared by
+// all XCDs, about 12 us, whatever it carries: one entry per donation took 13.5
+// ms for three graphs of n = 225..250 with half of all edges and 34.4 ms for
+// two of n = 180..200 and mean degree 10, up to four take 11.9 and 30.1.
+constexpr uint32_t kDonateBatch = 4;
+__device__ __forceinline__ bool try_enqueue_bits(const SolveArgs &a, uint32_t g, uint32_t ctx, uint32_t words, uint32_t count,
+                                                 const char *stk, const uint2 *stk_meta, uint32_t bot, uint32_t slot_bytes)
 {
-    uint32_t slot, ticket;
-    if (!reserve_slot(a, g, slot, ticket)) return false;
-    if (lane_id() < words)
-        __builtin_amdgcn_raw_buffer_store_b32(word, slot_rsrc(static_cast<char *>(a.q_deg) + (size_t)slot * slot_bytes, slot_bytes),
-                                              4u * lane_id(), 0, kCoherent);
-    publish_slot(a, slot, ticket, u32x4{g, d, words, ctx + 1u});
+    const uint32_t lane = lane_id(), e = lane / 16u;
+    uint32_t word = 0, d = 0;
+    if (e < count) word = reinterpret_cast<const uint32_t *>(stk + (size_t)((bot + e) % a.depth) * slot_bytes)[lane % 16u];
+    if (lane < count) d = stk_meta[(bot + lane) % a.depth].x;
+    uint32_t ok = 1, lo = 0, hi = 0;
+    if (lane == 0) {
+        if (a.ring_guard && fetch_add(&a.glob->count, (int)count) + (int)count > (int)a.qsize) {
+            fetch_add(&a.glob->count, -(int)count);
+            ok = 0;
+        } else {
+            const unsigned long long pos = fetch_add(&a.glob->tail, (unsigned long long)count);
+            lo = (uint32_t)pos;
+            hi = (uint32_t)(pos >> 32);
+        }
+    }
+    if (!uni(ok)) return false;
+    const unsigned long long first = ((unsigned long long)uni(hi) << 32) | uni(lo);
+    const unsigned long long pos = first + lane;
+    const uint32_t slot = (uint32_t)(pos & (unsigned long long)(a.qsize - 1)), ticket = (uint32_t)(2ull * (pos / a.qsize));
+    // the slots are free once their previous consumers have stored 2 lap
+    for (uint32_t spins = 0;; ++spins) {
+        const bool wait = lane < count && ld_rlx(&a.tickets[slot]) != ticket;
+        if (__ballot(wait) == 0ull) break;
+        backoff(spins < 3 ? spins : 3);
+        uint32_t late = 0;
+        if (lane == 0) late = past_deadline(a);
+        if (uni(late)) return false;  // the launch is being cancelled: leave the slots alone
+    }
+    if (lane == 0) fetch_add(&a.gstate[g].outstanding, count);
+    handoff_observe();
+    const uint32_t my_slot = (uint32_t)((first + e) & (unsigned long long)(a.qsize - 1));
+    if (e < count && lane % 16u < words) {
+        uint32_t *const to = reinterpret_cast<uint32_t *>(static_cast<char *>(a.q_deg) + (size_t)my_slot * slot_bytes) + lane % 16u;
+        __hip_atomic_store(to, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (lane < count) {
+        const u32x4 m = {g, d, words, ctx + 1u};
+        uint32_t *const to = reinterpret_cast<uint32_t *>(&a.q_meta[slot]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) __hip_atomic_store(to + q, m[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    handoff_publish();
+    if (lane < count) st_rlx(&a.tickets[slot], ticket + 1u);
+    if (lane == 0) fetch_add(&a.glob->counter, (unsigned long long)count * kEnqOne);
     return true;
 }
 
@@ -1336,17 +1379,18 @@ __device__ __forceinline__ uint32_t next_random(uint32_t &state)
 // Should this worker donate, given the launch's counter?  While workers wait
 // and the worklist holds fewer items than there are waiting workers (and
 // fewer than the -t threshold).  Of the many busy workers that see the same
-// shortage only about twice as many as items are missing act on it: when all
+// shortage only about twice as many as items are missing act on it (returns how
+// many are missing, 0 = do not donate): when all
 // did, a search of 470,000 nodes on 4,096 workers made 183,000 donations and
 // took 48 ms, against 17 ms on 1,024 workers.
-__device__ __forceinline__ bool wants_donation(const SolveArgs &a, unsigned long long counter, uint32_t &rnd)
+__device__ __forceinline__ uint32_t wants_donation(const SolveArgs &a, unsigned long long counter, uint32_t &rnd)
 {
     const uint32_t lo = uni((uint32_t)counter), enq = (uint32_t)max((int)uni((uint32_t)(counter >> 32)), 0);
     const uint32_t waiting = lo & 0xFFFFu, busy = (lo >> 16) - waiting;
-    if (waiting == 0u || enq >= waiting || enq >= a.qthreshold) return false;
-    const uint32_t missing = waiting - enq;
-    if (2u * missing >= busy) return true;
-    return ((next_random(rnd) * busy) >> 16) < 2u * missing;
+    if (waiting == 0u || enq >= waiting || enq >= a.qthreshold) return 0u;
+    const uint32_t missing = min(waiting, a.qthreshold) - enq;
+    if (2u * missing >= busy) return missing;
+    return ((next_random(rnd) * busy) >> 16) < 2u * missing ? missing : 0u;
 }
 
 // Takes the next item of the ring; the caller has taken one off the
@@ -2231,7 +2275,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         // then goes from the node storage straight to the worklist (a
         // BA n = 2,000 search, a chain of nodes that each donate their
         // right child, took 0.93 ms with the copy through the stack).
-        const bool donate = a.version == 1 && wants_donation(a, ld_rlx(&a.glob->counter), rnd);
+        const bool donate = a.version == 1 && wants_donation(a, ld_rlx(&a.glob->counter), rnd) != 0u;
         if (donate && top < bot && uni(try_enqueue(a, w, w.base, g, d, v, slot_bytes)) != 0u) {
             ++donations;
             moved += copy_bytes<NodeT>(w.n);
@@ -3057,7 +3101,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
         if ((p->list_size & (p->list_size - 1u)) != 0u) return VC_EINVAL;
         pl.qsize = p->list_size;
     } else {
-        pl.qsize = next_pow2(std::max<uint32_t>(1024u, 2u * pl.workers));
+        pl.qsize = next_pow2(std::max<uint32_t>(1024u, 8u * pl.workers));
     }
     if (p->list_threshold > 0.f) {
         pl.qthreshold = (uint32_t)(p->list_threshold * (float)pl.qsize);
@@ -3161,7 +3205,7 @@ void fill_args(SolveArgs &a, const Plan &pl, char *base, uint32_t version, uint3
     a.depth = pl.depth;
     a.qsize = pl.qsize;
     a.qthreshold = pl.qthreshold;
-    a.ring_guard = pl.qsize < 2u * pl.workers;
+    a.ring_guard = pl.qsize < 6u * pl.workers;
     a.workers = pl.workers;
     a.version = version;
     a.start_depth = version == VC_STACK_ONLY ? start_depth : 0u;

@@ -47,3 +47,18 @@ def test_context_sizes_match_oracle(ctx, n, version):
                 continue
             assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)), (name, n)
             assert int(np.sum(r.cover)) == want, (name, n)
+
+
+@pytest.mark.parametrize("list_size", [1, 2, 4, 64, 4096, 8192])
+def test_donated_batches_fit_any_ring(ctx, list_size):
+    """Donations of several stack entries into rings smaller than a batch,
+    smaller than the launch's workers need, and large enough never to fill."""
+    params = vcgpu.Params(list_size=list_size, time_limit_ms=60000)
+    for e, n in ((graphgen.erdos_renyi(110, 0.5, 61), 110), (graphgen.erdos_renyi(100, 0.06, 62), 100)):
+        og = O.from_edges(n, e)
+        want, stats, _ = O.mvc(og, max_nodes=2_000_000)
+        assert stats["completed"]
+        gs = ctx.upload([vcgpu.csr_from_edges(n, e)])
+        (r,), info, st = ctx.solve(gs, [vcgpu.Job(vcgpu.VC_MVC, 0, n - 1, 0)], params)
+        assert st == vcgpu.VC_OK and r.solved and r.minimum == want
+        assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == want
