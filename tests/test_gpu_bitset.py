@@ -62,3 +62,22 @@ def test_donated_batches_fit_any_ring(ctx, list_size):
         (r,), info, st = ctx.solve(gs, [vcgpu.Job(vcgpu.VC_MVC, 0, n - 1, 0)], params)
         assert st == vcgpu.VC_OK and r.solved and r.minimum == want
         assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == want
+
+
+@pytest.mark.parametrize("p", [0.2, 0.25, 0.3, 0.5, 0.7])
+def test_densities_around_the_branch_rule_match_oracle(ctx, p):
+    """Remainders on both sides of a quarter of all edges, where the search
+    changes from a few branch vertices to all that the cliques leave over."""
+    n = 60
+    e = graphgen.erdos_renyi(n, p, int(700 + 100 * p))
+    og = O.from_edges(n, e)
+    want, stats, _ = O.mvc(og, max_nodes=2_000_000)
+    assert stats["completed"]
+    gs = ctx.upload([vcgpu.csr_from_edges(n, e)] * 3)
+    jobs = [vcgpu.Job(vcgpu.VC_MVC, 0, n - 1, 0), vcgpu.Job(vcgpu.VC_PVC, want - 1, n - 1, 0),
+            vcgpu.Job(vcgpu.VC_PVC, want, n - 1, 0)]
+    (mvc, no, yes), _, st = ctx.solve(gs, jobs, vcgpu.Params(time_limit_ms=60000))
+    assert st == vcgpu.VC_OK
+    assert mvc.solved and mvc.minimum == want and int(np.sum(mvc.cover)) == want
+    assert O.cover_is_valid(og, np.asarray(mvc.cover, np.uint8))
+    assert no.solved and not no.k_found and yes.solved and yes.k_found
