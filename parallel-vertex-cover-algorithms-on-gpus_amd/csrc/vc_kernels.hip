@@ -2739,6 +2739,14 @@ using vcg::GState;
 using vcg::Global;
 using vcg::SolveArgs;
 
+// Memory of a graph set: device memory, or pinned host memory that kernels
+// write.
+struct Block {
+    char *p = nullptr;
+    size_t bytes = 0;
+    bool host = false;
+};
+
 struct vc_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -2763,6 +2771,7 @@ struct vc_ctx {
     std::mutex mem_mu;
     int active_servers = 0;
     std::vector<std::pair<void *, bool>> deferred;  // (pointer, pinned host memory)
+    std::vector<Block> spare;                       // blocks of freed sets (take_block)
 };
 
 void free_now(void *p, bool host)
@@ -2785,6 +2794,53 @@ void ctx_release(vc_ctx *ctx, void *p, bool host)
         }
     }
     free_now(p, host);
+}
+
+// A block of at least `bytes` for a graph set: a spare one of a set freed
+// before, else a new one.  A program that asks about one small graph after the
+// other uploads, solves and frees a set per question, and allocating and
+// freeing its eight buffers was half of such a call (four graphs of n = 36..40:
+// 1.12 ms with them, 0.53 now).  A spare block is never in use: a solve
+// returns after its last kernel.  At most kSpareBlocks of kSpareBytes each are
+// kept, until the context is destroyed; larger ones are freed with their set.
+constexpr size_t kSpareBytes = 1u << 20;
+constexpr size_t kSpareBlocks = 8;
+bool take_block(vc_ctx *ctx, size_t bytes, bool host, Block &out)
+{
+    size_t size = 1u << 14;
+    while (size < bytes && size < kSpareBytes) size *= 2;
+    size = std::max(size, bytes);
+    if (size <= kSpareBytes) {
+        std::lock_guard<std::mutex> lk(ctx->mem_mu);
+        for (Block &b : ctx->spare)
+            if (b.host == host && b.bytes == size) {
+                out = b;
+                b = ctx->spare.back();
+                ctx->spare.pop_back();
+                return true;
+            }
+    }
+    void *p = nullptr;
+    const hipError_t e = host ? hipHostMalloc(&p, size, hipHostMallocCoherent | hipHostMallocMapped) : hipMalloc(&p, size);
+    if (e != hipSuccess) return false;
+    out = Block{static_cast<char *>(p), size, host};
+    return true;
+}
+
+// Keeps b (of a set on `device`) for a later set, or frees it.
+void give_block(vc_ctx *ctx, int device, Block &b)
+{
+    const Block x = b;
+    b = Block{};
+    if (!x.p) return;
+    if (ctx && ctx->device == device && x.bytes <= kSpareBytes) {
+        std::lock_guard<std::mutex> lk(ctx->mem_mu);
+        if (ctx->spare.size() < kSpareBlocks) {
+            ctx->spare.push_back(x);
+            return;
+        }
+    }
+    ctx_release(ctx, x.p, x.host);
 }
 
 // Releases the deferred frees once no server runs.
@@ -2840,6 +2896,10 @@ struct vc_graphs {
     int count = 0;
     vc_graphs *rest = nullptr;    // what shrink_kernel leaves of the set (buffers kept across solves)
     bool borrowed = false;        // d_words belongs to the context
+    int device = 0;
+    Block dev;                    // d_words, d_desc, d_covers and d_state
+    Block pinned;                 // h_state, h_glob and h_cov
+    Block stats;                  // h_ws
     bool dirty = false;           // h_desc differs from d_desc beyond the job fields
     uint32_t *h_shrink = nullptr; // pinned: old ids and cover bitmaps of shrink_kernel
     uint32_t leaf_share = 0;      // the least share of degree-1 vertices in a graph of the set, in 1/1024
@@ -2851,7 +2911,7 @@ struct vc_graphs {
     uint32_t nmax = 0;
     uint32_t cover_words = 0;
     double mean_n = 0, mean_density = 0;  // autotuner bucket
-    // pinned readback buffers (stable addresses, so a captured dispatch can
+    // readback buffers (stable addresses, so a captured dispatch can
     // copy into them on every replay)
     GState *h_state = nullptr;
     Global *h_glob = nullptr;
@@ -2869,6 +2929,23 @@ namespace {
 inline bool hip_ok(hipError_t e) { return e == hipSuccess; }
 
 inline uint32_t round_up(uint32_t x, uint32_t m) { return (x + m - 1) / m * m; }
+
+inline size_t block_up(size_t bytes) { return (bytes + 255u) / 256u * 256u; }
+
+// The set's device memory: `words` words of CSR arrays (0: they are the
+// context's), descriptors, cover bitmaps and graph states.
+bool take_device(vc_ctx *ctx, vc_graphs *s, size_t words)
+{
+    const size_t csr = block_up(sizeof(uint32_t) * words), desc = block_up(sizeof(GDesc) * (size_t)s->count);
+    const size_t cov = block_up(sizeof(uint32_t) * (size_t)s->cover_words);
+    s->device = ctx->device;
+    if (!take_block(ctx, csr + desc + cov + sizeof(GState) * (size_t)s->count, false, s->dev)) return false;
+    if (words) s->d_words = reinterpret_cast<uint32_t *>(s->dev.p);
+    s->d_desc = reinterpret_cast<GDesc *>(s->dev.p + csr);
+    s->d_covers = reinterpret_cast<uint32_t *>(s->dev.p + csr + desc);
+    s->d_state = reinterpret_cast<GState *>(s->dev.p + csr + desc + cov);
+    return true;
+}
 
 inline uint32_t next_pow2(uint32_t x)
 {
@@ -3331,6 +3408,7 @@ vc_status vc_ctx_destroy(vc_ctx *c)
     if (c->scratch) (void)hipFree(c->scratch);
     if (c->shrink_work) (void)hipFree(c->shrink_work);
     if (c->shrink_io) (void)hipHostFree(c->shrink_io);
+    for (Block &b : c->spare) free_now(b.p, b.host);
     for (auto &x : c->deferred) free_now(x.first, x.second);
     c->deferred.clear();
     if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -3412,13 +3490,14 @@ vc_status vc_graphs_upload(vc_ctx *ctx, int count, const vc_csr *graphs, vc_grap
                     host[d.off_bits + (bit >> 5)] |= 1u << (bit & 31u);
                 }
     }
-    bool ok = hip_ok(hipMalloc(&s->d_words, host.size() * sizeof(uint32_t))) &&
-              hip_ok(hipMalloc(&s->d_desc, sizeof(GDesc) * count)) &&
-              hip_ok(hipMalloc(&s->d_covers, sizeof(uint32_t) * s->cover_words)) &&
-              hip_ok(hipMalloc(&s->d_state, sizeof(GState) * count));
-    if (ok)
-        ok = hip_ok(hipMemcpy(s->d_words, host.data(), host.size() * sizeof(uint32_t), hipMemcpyHostToDevice)) &&
-             hip_ok(hipMemcpy(s->d_desc, s->h_desc.data(), sizeof(GDesc) * count, hipMemcpyHostToDevice));
+    // the descriptors follow the CSR arrays: one copy
+    bool ok = take_device(ctx, s, host.size());
+    if (ok) {
+        host.resize(block_up(sizeof(uint32_t) * host.size()) / sizeof(uint32_t) + sizeof(GDesc) / sizeof(uint32_t) * (size_t)count);
+        std::memcpy(host.data() + host.size() - sizeof(GDesc) / sizeof(uint32_t) * (size_t)count, s->h_desc.data(),
+                    sizeof(GDesc) * (size_t)count);
+        ok = hip_ok(hipMemcpy(s->d_words, host.data(), host.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    }
     if (!ok) {
         vc_graphs_free(ctx, s);
         return VC_ENOMEM;
@@ -3432,17 +3511,12 @@ vc_status vc_graphs_free(vc_ctx *ctx, vc_graphs *s)
     if (!s) return VC_EINVAL;
     if (ctx) (void)hipSetDevice(ctx->device);
     if (s->rest) vc_graphs_free(ctx, s->rest);
-    if (!s->borrowed) ctx_release(ctx, s->d_words, false);
-    ctx_release(ctx, s->h_shrink, true);
-    ctx_release(ctx, s->d_desc, false);
-    ctx_release(ctx, s->d_covers, false);
-    ctx_release(ctx, s->d_state, false);
-    ctx_release(ctx, s->h_state, true);
-    ctx_release(ctx, s->h_glob, true);
-    ctx_release(ctx, s->h_ws, true);
-    ctx_release(ctx, s->h_cov, true);
     if (s->exec) (void)hipGraphExecDestroy(s->exec);
     if (s->graph) (void)hipGraphDestroy(s->graph);
+    ctx_release(ctx, s->h_shrink, true);
+    give_block(ctx, s->device, s->dev);
+    give_block(ctx, s->device, s->pinned);
+    give_block(ctx, s->device, s->stats);
     delete s;
     return VC_OK;
 }
@@ -3588,20 +3662,22 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
     bool want_covers = false;
     if (covers)
         for (int i = 0; i < set->count; ++i) want_covers |= covers[i] != nullptr;
-    // pinned readback buffers, mapped: publish_kernel writes them
-    constexpr unsigned kPinned = hipHostMallocCoherent | hipHostMallocMapped;
-    bool ok = true;
-    if (!set->h_state)
-        ok = hip_ok(hipHostMalloc(reinterpret_cast<void **>(&set->h_state), sizeof(GState) * set->count, kPinned)) &&
-             hip_ok(hipHostMalloc(reinterpret_cast<void **>(&set->h_glob), sizeof(Global), kPinned)) &&
-             hip_ok(hipHostMalloc(reinterpret_cast<void **>(&set->h_cov), sizeof(uint32_t) * set->cover_words, kPinned));
-    if (ok && set->ws_cap < pl.workers) {
-        ctx_release(ctx, set->h_ws, true);
-        set->h_ws = nullptr;
-        ok = hip_ok(hipHostMalloc(reinterpret_cast<void **>(&set->h_ws), sizeof(vcg::WorkerStats) * pl.workers, kPinned));
-        set->ws_cap = ok ? pl.workers : 0;
+    // readback buffers, pinned and mapped: publish_kernel writes them
+    if (!set->h_state) {
+        const size_t state = block_up(sizeof(GState) * (size_t)set->count), glob = block_up(sizeof(Global));
+        if (!take_block(ctx, state + glob + sizeof(uint32_t) * (size_t)set->cover_words, true, set->pinned)) return VC_ENOMEM;
+        set->h_state = reinterpret_cast<GState *>(set->pinned.p);
+        set->h_glob = reinterpret_cast<Global *>(set->pinned.p + state);
+        set->h_cov = reinterpret_cast<uint32_t *>(set->pinned.p + state + glob);
     }
-    if (!ok) return VC_ENOMEM;
+    if (set->ws_cap < pl.workers) {
+        give_block(ctx, set->device, set->stats);
+        set->h_ws = nullptr;
+        set->ws_cap = 0;
+        if (!take_block(ctx, sizeof(vcg::WorkerStats) * (size_t)pl.workers, true, set->stats)) return VC_ENOMEM;
+        set->h_ws = reinterpret_cast<vcg::WorkerStats *>(set->stats.p);
+        set->ws_cap = pl.workers;
+    }
 
     // the device work of one solve, in stream order
     auto enqueue_dispatch = [&](bool timed) -> bool {
@@ -3830,9 +3906,7 @@ static vc_status solve_shrunk(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, c
             rest->borrowed = true;
             rest->h_desc = set->h_desc;
             rest->cover_words = set->cover_words;
-            if (!hip_ok(hipMalloc(&rest->d_desc, sizeof(GDesc) * count)) ||
-                !hip_ok(hipMalloc(&rest->d_covers, sizeof(uint32_t) * rest->cover_words)) ||
-                !hip_ok(hipMalloc(&rest->d_state, sizeof(GState) * count))) {
+            if (!take_device(ctx, rest, 0)) {
                 vc_graphs_free(ctx, rest);
                 return VC_ENOMEM;
             }
