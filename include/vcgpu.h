@@ -60,7 +60,8 @@ typedef struct {
     uint32_t k;           /* PVC parameter (-k, src/config.h:211-213) */
     uint32_t upper_bound; /* U; must be the size of some vertex cover */
     uint32_t reserved;
-    uint64_t max_nodes;   /* per-graph tree-node budget, 0 = unlimited; a graph that reaches
+    uint64_t max_nodes;   /* per-graph tree-node budget, 0 = unlimited (and then with the
+                             bitset search, whose nodes are fewer and dearer); a graph that reaches
                              it stops within a few percent of it (workers flush their node
                              counts more often as the budget runs out) and reports
                              VC_ETIMEOUT with its incumbent */
@@ -74,10 +75,11 @@ typedef struct {
                                    one search worker per 64-thread wave; 0 = auto.  When an
                                    explicit workgroup's workers do not fit in LDS their node
                                    state goes to HBM (as with -g 1) */
-    uint32_t num_blocks;        /* workgroups (-n); 0 = auto (occupancy x CUs).  At most
+    uint32_t num_blocks;        /* workgroups (-n); 0 = auto (one worker per SIMD; as many as
+                                   fit when every graph has a node budget).  At most
                                    65535 workers (num_blocks x block_dim / 64) per launch.
                                    With 0 and fewer roots (graphs x static paths) than half
-                                   the workers, 512 workers start and the rest join once
+                                   the workers, 256 (512) workers start and the rest join once
                                    they are nearly all busy and the launch has run 0.8 ms
                                    (a small search ends before they do); an explicit
                                    num_blocks starts every worker at once */
@@ -140,7 +142,8 @@ typedef struct {
     uint64_t state_bytes; /* HBM bytes of node state the search moved: every stack
                              push and pop, worklist steal, and (twice) donation copies
                              the graph's degree/sketch records, 8 bytes per vertex (16
-                             in the int32 layout) in 16-byte vectors; 0 from a server */
+                             in the int32 layout) in 16-byte vectors, or in the bitset
+                             search its masks (16 bytes per 64 vertices); 0 from a server */
 } vc_launch_info;
 
 typedef struct vc_ctx vc_ctx;

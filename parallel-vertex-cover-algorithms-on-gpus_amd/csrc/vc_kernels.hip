@@ -203,7 +203,8 @@ __device__ __forceinline__ void backoff(uint32_t step, uint32_t cap = 6u)
 // Sleep of an idle worker between polls of the worklist.  Every poll reads
 // launch-wide words that all workers share, so with thousands of idle
 // workers the polls themselves slow down the few busy ones (a search of
-// 5,000 tree nodes took 4.2 ms on 7,168 workers and 0.57 ms on 512).  The
+// 5,000 tree nodes without the bitset search took 4.2 ms on 7,168 workers and
+// 0.57 ms on 512).  The
 // interval therefore grows with the number of waiting workers -- about one
 // s_sleep(8) unit (~0.2 us) per 16 of them, i.e. a fixed total poll rate --
 // with a jitter from the clock's low bits so that workers that went idle
@@ -1822,8 +1823,8 @@ __device__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes,
 
 // Staged start.  A launch with few roots (one graph, a handful) cannot use
 // thousands of workers at first, and idle workers are not free: every one
-// polls the launch-wide words, and a 5,000-node search took 4.2 ms on 7,168
-// workers but 0.5 ms on 256.  So only workers wid < active0 start at once;
+// polls the launch-wide words, and a 5,000-node general search took 4.2 ms on
+// 7,168 workers but 0.5 ms on 256.  So only workers wid < active0 start at once;
 // the others sleep, then look at the pool: once the launch has run for
 // 8 x dormant_ticks they join (register and look for work) while at most
 // one in eight registered workers waits, and otherwise sleep again, for
@@ -1936,7 +1937,7 @@ namespace vcg {
 // The kernel body takes the launch arguments by reference from a one-line
 // kernel: hipcc then allocates 55 instead of 81 VGPRs for the int16 LDS
 // variant (same source otherwise), so the LDS budget alone sets occupancy.
-template <typename DegT, bool HBM, bool SERVE, bool OFF16, bool STAGED, bool ADJ = false>
+template <typename DegT, bool HBM, bool SERVE, bool OFF16, bool STAGED, bool ADJ = false, bool BITS = true>
 __device__ __forceinline__ void solve_body(const SolveArgs &a)
 {
     extern __shared__ int4 smem4[];
@@ -2110,7 +2111,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     cands_reset(c, q.v == kNone);
                     if (q.v != kNone) d += take_neighbours(w, q.v, c);
                     descend = 0;
-                } else if (a.version == 1 && w.n - 1u < a.bits_max) {
+                } else if (BITS && a.version == 1 && gd.max_nodes == 0u && w.n - 1u < a.bits_max) {
                     // a small graph needs no node state: its rows straight
                     // from the adjacency, its first reductions on masks
                     d = 0;
@@ -2196,7 +2197,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 }
                 continue;
             }
-            if (s.live <= a.bits_max) {
+            if (BITS && gd.max_nodes == 0u && s.live <= a.bits_max) {
                 bits = s.live;
             } else if (s.maxdeg <= 2) {
                 // cycles only: some minimum cover holds v
@@ -2205,7 +2206,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 continue;
             }
         }
-        if (bits != 0u || bits_ctx != kNone) {
+        if constexpr (BITS) if (bits != 0u || bits_ctx != kNone) {
             BitsWorker bw;
             bw.stk = stk;
             bw.stk_meta = stk_meta;
@@ -2677,14 +2678,24 @@ __global__ __launch_bounds__(1024) void solve_kernel(SolveArgs a)
 
 template __global__ void solve_kernel<int16_t, false, false>(SolveArgs);
 // Batch launches whose graphs all have 2m < 2^16 keep each worker's current
-// srcPtr in LDS (OFF16).  Asking for 7 waves per SIMD caps the body at 72
-// VGPRs (about 40 spilled, mostly off the per-node path); with 64-entry
-// candidate lists a worker's LDS at n = 400 lets 28 workers share a CU.
-// Measured per batched step: 2.87 s at 7 waves against 3.16 s at 6 (80
-// VGPRs) and 3.38 s at 8 (64 VGPRs, 68 spilled).
+// srcPtr in LDS (OFF16).  Workgroups of up to 1,024 threads put four waves on
+// a SIMD, so a wave has 128 VGPRs; more waves with fewer registers would serve
+// nothing, a launch has one worker per SIMD (kSolveWorkersPerCU).
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void solve_kernel_off16(SolveArgs a)
 {
     solve_body<int16_t, false, false, true, false>(a);
+}
+// Launches in which every graph has a node budget (searches_nodes): no bitset
+// search, so 7 waves per SIMD and 72 VGPRs (about 40 spilled, mostly off the
+// per-node path).  Per batched step: 2.87 s at 7 waves against 3.16 s at 6 (80
+// VGPRs) and 3.38 s at 8 (64 VGPRs, 68 spilled).
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void solve_kernel_off16_nodes(SolveArgs a)
+{
+    solve_body<int16_t, false, false, true, false, false, false>(a);
+}
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void solve_kernel_off16_staged_nodes(SolveArgs a)
+{
+    solve_body<int16_t, false, false, true, true, false, false>(a);
 }
 // The same with a staged start (launches with few roots, dormant_join).
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void solve_kernel_off16_staged(SolveArgs a)
@@ -2990,7 +3001,7 @@ bool csr_is_valid(const vc_csr &g)
 // need at least 512 KB at n = 32768, so they are never LDS-resident.
 enum Variant { kLds16 = 0, kHbm16 = 1, kHbm32 = 2 };
 
-const void *kernel_of(int variant, bool serve, bool off16 = false, bool adj = false)
+const void *kernel_of(int variant, bool serve, bool off16 = false, bool adj = false, bool nodes = false)
 {
     if (adj) return reinterpret_cast<const void *>(vcg::solve_kernel_off16_adj);
     if (serve) {
@@ -3002,7 +3013,7 @@ const void *kernel_of(int variant, bool serve, bool off16 = false, bool adj = fa
     }
     switch (variant) {
     case kLds16:
-        return off16 ? reinterpret_cast<const void *>(vcg::solve_kernel_off16)
+        return off16 ? reinterpret_cast<const void *>(nodes ? vcg::solve_kernel_off16_nodes : vcg::solve_kernel_off16)
                      : reinterpret_cast<const void *>(vcg::solve_kernel<int16_t, false, false>);
     case kHbm16: return reinterpret_cast<const void *>(vcg::solve_kernel<int16_t, true, false>);
     default: return reinterpret_cast<const void *>(vcg::solve_kernel<int32_t, true, false>);
@@ -3016,6 +3027,7 @@ struct Plan {
     uint32_t depth, qsize, qthreshold, roots, units;
     uint32_t off16;  // workers keep their graph's srcPtr in LDS as uint16
     uint32_t adj;    // ... and its dst (solve_kernel_off16_adj, a staged launch)
+    uint32_t nodes;  // no bitset search (searches_nodes)
     size_t smem;
     size_t off_glob, off_stk, off_meta, off_qdeg, off_qmeta, off_tickets, off_wnodes, off_ctx, off_hbm, total;
 };
@@ -3062,7 +3074,7 @@ void size_storage(Plan &pl, uint32_t nmax, uint32_t deg_bytes, bool off16 = fals
 
 // LDS of a worker's contexts, and of a workgroup of wpb workers with their
 // node storage in LDS.
-uint32_t bits_lds(const Plan &pl) { return pl.bits_max == vcg::kBitsMax ? vcg::kCtxLdsBytes : vcg::kCtxLdsSmall; }
+uint32_t bits_lds(const Plan &pl) { return pl.bits_max == 0u ? 0u : pl.bits_max == vcg::kBitsMax ? vcg::kCtxLdsBytes : vcg::kCtxLdsSmall; }
 size_t lds_bytes(const Plan &pl, uint32_t wpb) { return (size_t)wpb * (bits_lds(pl) + pl.worker_bytes); }
 
 // Launch shape shared by the batch solve and the server: node storage,
@@ -3078,7 +3090,7 @@ constexpr uint32_t kMaxBlockDim = 1024;   // the solve kernels' launch bound
 constexpr uint32_t kMaxWorkers = 0xFFFFu; // 16-bit worker counts in the termination word
 
 vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_params *p, Plan &pl, bool serve,
-                      bool off16_ok = false, size_t mem_budget = 0, uint32_t adj_entries = 0)
+                      bool off16_ok = false, size_t mem_budget = 0, uint32_t adj_entries = 0, bool nodes = false)
 {
     const uint32_t version = p->version;
     if (version != VC_HYBRID && version != VC_STACK_ONLY) return VC_EINVAL;
@@ -3098,7 +3110,8 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     // -g 0 forbids it); int16 degrees while n < 32768 (VC_FLAG_WIDE forces
     // int32).
     const bool wide = nmax >= 32768u || (p->flags & VC_FLAG_WIDE) != 0u;
-    pl.bits_max = vcg::kBitsMax;
+    pl.nodes = nodes;
+    pl.bits_max = nodes ? 0u : vcg::kBitsMax;
     size_storage(pl, nmax, wide ? 4u : 2u);
     uint32_t wpb = block_dim / vcg::kWave;
     bool hbm = wide || p->use_global_memory == 1;
@@ -3106,7 +3119,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
         if (!p->block_dim)
             while (wpb > 1 && lds_bytes(pl, wpb) > lds_limit) wpb /= 2;
         // an explicit workgroup whose workers fit with smaller contexts only
-        if (lds_bytes(pl, wpb) > lds_limit) pl.bits_max = vcg::kBitsMaxSmall;
+        if (!nodes && lds_bytes(pl, wpb) > lds_limit) pl.bits_max = vcg::kBitsMaxSmall;
         hbm = lds_bytes(pl, wpb) > lds_limit;
     }
     if (hbm && p->use_global_memory == 0) return VC_ENOTSUP;
@@ -3141,12 +3154,13 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     }
     pl.wpb = wpb;
     pl.block_dim = wpb * vcg::kWave;
-    if (hbm) pl.bits_max = (size_t)wpb * vcg::kCtxLdsBytes <= lds_limit ? vcg::kBitsMax : vcg::kBitsMaxSmall;
-    pl.smem = (size_t)pl.wpb * (bits_lds(pl) + (hbm ? 0u : pl.worker_bytes));
+    if (hbm && !nodes) pl.bits_max = (size_t)wpb * vcg::kCtxLdsBytes <= lds_limit ? vcg::kBitsMax : vcg::kBitsMaxSmall;
+    // (a staged start shares one word of LDS)
+    pl.smem = std::max<size_t>(16u, (size_t)pl.wpb * (bits_lds(pl) + (hbm ? 0u : pl.worker_bytes)));
     if (pl.smem > lds_limit) return VC_ENOTSUP;
 
     int bpc = 0;
-    if (!hip_ok(hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, kernel_of(pl.variant, serve, pl.off16 != 0u, pl.adj != 0u),
+    if (!hip_ok(hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, kernel_of(pl.variant, serve, pl.off16 != 0u, pl.adj != 0u, nodes),
                                                              (int)pl.block_dim, pl.smem)))
         return VC_EDEVICE;
     if (bpc < 1) return VC_ENOTSUP;
@@ -3161,7 +3175,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
         // occupancy grid a vc_solve issued beside a server waited for it.
         auto_blocks = std::min<uint32_t>(
             auto_blocks, std::max<uint32_t>(1u, kServeWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
-    } else {
+    } else if (!nodes) {
         auto_blocks = std::min<uint32_t>(
             auto_blocks, std::max<uint32_t>(1u, kSolveWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
     }
@@ -3218,6 +3232,20 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     return VC_OK;
 }
 
+// A node budget limits a search by its number of nodes, and most of a budgeted
+// launch's nodes are those of graphs that end at the budget.  A node of the
+// bitset search costs much more than one of the general search, and the
+// general search runs 28 workers per CU instead of four: 4,096 graphs with a
+// budget of 2^20 nodes each take 2.8 s (2,697 solved) against 17.0 s (2,895).
+// So graphs with a budget are searched without it, and a launch of only such
+// graphs keeps no contexts in LDS and fills the SIMDs.
+bool searches_nodes(const vc_graphs *set, const vc_job *jobs)
+{
+    for (int i = 0; i < set->count; ++i)
+        if (jobs[i].max_nodes == 0u) return false;
+    return true;
+}
+
 vc_status make_plan(vc_ctx *ctx, const vc_graphs *set, const vc_job *jobs, const vc_params *p, Plan &pl,
                     size_t mem_budget = 0)
 {
@@ -3236,7 +3264,8 @@ vc_status make_plan(vc_ctx *ctx, const vc_graphs *set, const vc_job *jobs, const
         off16_ok &= 2ull * set->h_desc[i].m < 65536ull;
         e2max = std::max<uint32_t>(e2max, (uint32_t)std::min<uint64_t>(2ull * set->h_desc[i].m, 0xFFFFFFFFull));
     }
-    vc_status st = plan_launch(ctx, set->nmax, need + 1u, p, pl, false, off16_ok, mem_budget);
+    const bool nodes = searches_nodes(set, jobs);
+    vc_status st = plan_launch(ctx, set->nmax, need + 1u, p, pl, false, off16_ok, mem_budget, 0u, nodes);
     if (st != VC_OK) return st;
     // A launch of few roots on the automatic grid (the staged start) also
     // tries the adjacency in LDS (solve_kernel_off16_adj).  Taken when it
@@ -3247,7 +3276,7 @@ vc_status make_plan(vc_ctx *ctx, const vc_graphs *set, const vc_job *jobs, const
     const uint64_t roots_est = (uint64_t)set->count * pl.units;
     if (!p->num_blocks && pl.off16 && e2max > 0 && 2ull * roots_est < pl.workers) {
         Plan pa;
-        if (plan_launch(ctx, set->nmax, need + 1u, p, pa, false, off16_ok, mem_budget, e2max) == VC_OK && pa.adj &&
+        if (plan_launch(ctx, set->nmax, need + 1u, p, pa, false, off16_ok, mem_budget, e2max, nodes) == VC_OK && pa.adj &&
             (pa.workers >= pl.workers || set->nmax >= kAdjBitsMaxN))
             pl = pa;
     }
@@ -3303,7 +3332,10 @@ void launch_variant(const Plan &pl, hipStream_t stream, const SolveArgs &a)
         // staged start: the same kernels with the dormant_join prologue
         switch (pl.variant) {
         case kLds16:
-            if (pl.off16)
+            if (pl.off16 && pl.nodes)
+                hipLaunchKernelGGL(vcg::solve_kernel_off16_staged_nodes, dim3(pl.num_blocks), dim3(pl.block_dim), pl.smem,
+                                   stream, a);
+            else if (pl.off16)
                 hipLaunchKernelGGL(vcg::solve_kernel_off16_staged, dim3(pl.num_blocks), dim3(pl.block_dim), pl.smem,
                                    stream, a);
             else
@@ -3323,7 +3355,10 @@ void launch_variant(const Plan &pl, hipStream_t stream, const SolveArgs &a)
     }
     switch (pl.variant) {
     case kLds16:
-        if (!SERVE && pl.off16)
+        if (!SERVE && pl.off16 && pl.nodes)
+            hipLaunchKernelGGL(vcg::solve_kernel_off16_nodes, dim3(pl.num_blocks), dim3(pl.block_dim), pl.smem, stream,
+                               a);
+        else if (!SERVE && pl.off16)
             hipLaunchKernelGGL(vcg::solve_kernel_off16, dim3(pl.num_blocks), dim3(pl.block_dim), pl.smem, stream,
                                a);
         else
@@ -3578,17 +3613,16 @@ vc_status prepare_solve(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, const v
 }
 
 // Launch arguments of a batch solve of `set` with scratch at base.
-// Workers that start at once in a staged launch: two per CU.  Kernel time
-// with 128 / 256 / 512 starting workers (the rest joining as described at
-// dormant_join; measured before its end-only look, which took the 512 case
-// of the first graph to 0.64-0.66 ms): 3-regular n = 120 MVC (5,453 nodes) 0.73-0.74 / 0.66-0.67 /
-// 0.72-0.77 ms; BA n = 2,000 PVC answer 0.57 / 0.57 / 0.46 ms; ER
-// G(200, 0.05) MVC ~210 ms for all three.  256 helps only searches under a
-// millisecond (four 3-regular n = 120 graphs: 12-15%) and hurts longer ones
-// that still end before the others join (3-regular n = 160, 36k nodes:
-// 2.25 -> 3.3 ms; ER G(120, 0.08), 199k nodes: 14.9 -> 16.3 ms).  With every
-// worker started (7,168) the n = 120 search took 2.4-3.0 ms.
-constexpr uint32_t kActiveStart = 512;
+// Workers that start at once in a staged launch (the rest join as described at
+// dormant_join): one per CU.  With 128 / 256 / 512: four graphs of n = 36..40
+// 0.50 / 0.51 / 0.54 ms, four 3-regular graphs of n = 108..120 1.50 / 1.47 /
+// 1.52 ms, BA n = 2,000 PVC pair 0.85 / 0.86 / 0.88 ms, three graphs of n =
+// 225..250 with half of all edges 8.38 / 8.16 / 8.21 ms, two of n = 180..200,
+// mean degree 10, 30.9 / 31.4 / 30.2 ms (runs differ by 3%).  The general
+// search alone keeps two per CU: its searches are longer (3-regular n = 160,
+// 36k nodes: 2.25 ms with 512, 3.3 with 256).
+constexpr uint32_t kActiveStart = 256;
+constexpr uint32_t kActiveStartNodes = 512;
 
 SolveArgs solve_args(const vc_ctx *ctx, const vc_graphs *set, const vc_params *params, const Plan &pl, char *base)
 {
@@ -3606,8 +3640,9 @@ SolveArgs solve_args(const vc_ctx *ctx, const vc_graphs *set, const vc_params *p
     // staged start (vcg::dormant_join) when the grid is automatic and the
     // roots could keep fewer than half the workers busy; the adjacency
     // kernel is always staged (active0 >= workers: every worker starts)
-    if (pl.adj || (!params->num_blocks && 2ull * pl.roots < pl.workers && kActiveStart < pl.workers)) {
-        a.active0 = round_up(std::max<uint32_t>(kActiveStart, 2u * pl.roots), pl.wpb);
+    const uint32_t start = pl.nodes ? kActiveStartNodes : kActiveStart;
+    if (pl.adj || (!params->num_blocks && 2ull * pl.roots < pl.workers && start < pl.workers)) {
+        a.active0 = round_up(std::max<uint32_t>(start, 2u * pl.roots), pl.wpb);
         a.dormant_ticks = (uint64_t)ctx->wall_khz / 10u;  // 100 us
     }
     return a;
@@ -3711,7 +3746,7 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
         // The solve is bracketed by events outside the graph.
         DispatchKey key;
         std::memset(&key, 0, sizeof(key));
-        key.variant = pl.variant;
+        key.variant = pl.variant | (int)(pl.nodes << 8);
         key.num_blocks = pl.num_blocks;
         key.block_dim = pl.block_dim;
         key.version = a.version;
