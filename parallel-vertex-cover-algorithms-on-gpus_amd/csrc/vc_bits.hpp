@@ -297,12 +297,13 @@ __device__ __forceinline__ void load_rows(const BitsLds &lds, uint32_t level, Bi
 }
 
 // The remainder of the node in w (nq live vertices) into the LDS context of
-// `level`, in id order.  Positions of live vertices go to bytes over w.xs and
-// the candidate lists, which the subtree does not use.
+// `level`, in id order.  Positions of live vertices go to bytes over w.s2, which
+// the subtree does not use (of the node's state only the degrees' signs are read
+// again, for covers).
 template <int K, class N>
 __device__ __forceinline__ void build_rows(const N &w, const BitsLds &lds, uint32_t level, uint32_t nq)
 {
-    uint8_t *const pos = reinterpret_cast<uint8_t *>(w.xs);
+    uint8_t *const pos = reinterpret_cast<uint8_t *>(w.s2);
     uint32_t c = 0;
     w.sync();
     for (uint32_t base = 0, nv = uni(w.n); base < nv; base += kWave) {

@@ -2392,7 +2392,7 @@ __global__ void init_kernel(SolveArgs a, uint32_t units, uint32_t preload_roots)
     for (uint32_t i = tid; i < a.workers; i += stride) {
         a.wstats[i] = WorkerStats{};
         // users of the worker's contexts
-        for (uint32_t l = 0; l < kCtxLevels; ++l)
+        for (uint32_t l = 0; l < (a.ctx_bytes ? kCtxLevels : 0u); ++l)
             reinterpret_cast<uint32_t *>(a.ctx + (size_t)i * a.ctx_bytes)[l] = 0u;
     }
     if (tid == 0) {
@@ -3066,9 +3066,9 @@ void size_storage(Plan &pl, uint32_t nmax, uint32_t deg_bytes, bool off16 = fals
     pl.ncap = std::min<uint32_t>(round_up(nmax, 4u), adj_entries ? kCandCapLarge : cand_cap);
     const uint32_t id_bytes = deg_bytes == 2u ? 2u : 4u;  // mark and candidate list entries
     pl.mwords = round_up((nmax + 31u) / 32u, 4u);
-    // xs and the two candidate lists; vcg::build_rows keeps a byte per vertex there
-    pl.xs_bytes = std::max(4u * vcg::kWave + 2u * pl.ncap * id_bytes, round_up(pl.npad, 4u));
-    pl.ctx_bytes = vcg::kHbmCover + vcg::kCtxLevels * round_up(4u * round_up((nmax + 31u) / 32u, 2u), 128u);
+    pl.xs_bytes = 4u * vcg::kWave + 2u * pl.ncap * id_bytes;  // xs and the two candidate lists
+    // published contexts, where the search has any
+    pl.ctx_bytes = pl.bits_max ? vcg::kHbmCover + vcg::kCtxLevels * round_up(4u * round_up((nmax + 31u) / 32u, 2u), 128u) : 0u;
     pl.worker_bytes =
         round_up(pl.slot_bytes + id_bytes * pl.lcap + 4u * pl.mwords + pl.xs_bytes +
                      (off16 ? 2u * (pl.npad + 2u) : 0u) + 2u * round_up(adj_entries, 4u),
@@ -3092,8 +3092,8 @@ constexpr uint32_t kSolveWorkersPerCU = 4;
 constexpr uint32_t kMaxBlockDim = 1024;   // the solve kernels' launch bound
 constexpr uint32_t kMaxWorkers = 0xFFFFu; // 16-bit worker counts in the termination word
 
-vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_params *p, Plan &pl, bool serve,
-                      bool off16_ok = false, size_t mem_budget = 0, uint32_t adj_entries = 0, bool nodes = false)
+vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_params *p, Plan &pl, bool serve,
+                     bool off16_ok, size_t mem_budget, uint32_t adj_entries, bool nodes)
 {
     const uint32_t version = p->version;
     if (version != VC_HYBRID && version != VC_STACK_ONLY) return VC_EINVAL;
@@ -3190,18 +3190,12 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     pl.depth = std::max<uint32_t>(depth, 1u);
 
     // Worklist: size and donation threshold (-q, -t).
-    pl.workers = pl.num_blocks * pl.wpb;
-    if (p->list_size) {
-        if ((p->list_size & (p->list_size - 1u)) != 0u) return VC_EINVAL;
-        pl.qsize = p->list_size;
-    } else {
-        pl.qsize = next_pow2(std::max<uint32_t>(1024u, 8u * pl.workers));
-    }
-    if (p->list_threshold > 0.f) {
-        pl.qthreshold = (uint32_t)(p->list_threshold * (float)pl.qsize);
-    } else {
-        pl.qthreshold = pl.qsize;  // demand-driven: donate only while workers wait
-    }
+    if (p->list_size && (p->list_size & (p->list_size - 1u)) != 0u) return VC_EINVAL;
+    // An automatic worklist follows the grid as that shrinks: eight slots per
+    // worker, which donations of several entries cannot fill (reserve_slot), two
+    // without the bitset search.  (Sized once for the whole grid, 7,168 workers'
+    // ring of n = 400 alone was 208 MiB and vc_solve_noalloc refused the set.)
+    auto auto_ring = [&](uint32_t workers) { return next_pow2(std::max<uint32_t>(1024u, (nodes ? 2u : 8u) * workers)); };
 
     // Fit stacks + worklist into device memory; shrink the grid if needed
     // (the reference halves the worklist instead, src/auxFunctions.cpp:507-512).
@@ -3209,6 +3203,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
     const size_t budget = mem_budget ? mem_budget : ctx->total_mem / 10 * 7;
     for (;;) {
         pl.workers = pl.num_blocks * pl.wpb;
+        pl.qsize = p->list_size ? p->list_size : auto_ring(pl.workers);
         size_t off = 0;
         auto take = [&](size_t bytes) {
             size_t o = off;
@@ -3229,10 +3224,22 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_pa
         pl.num_blocks = std::max<uint32_t>(1u, pl.num_blocks / 2u);
     }
     if (pl.total > budget) return VC_ENOMEM;
+    // -t, or demand-driven: donate only while workers wait
+    pl.qthreshold = p->list_threshold > 0.f ? (uint32_t)(p->list_threshold * (float)pl.qsize) : pl.qsize;
 
     pl.units = version == VC_HYBRID ? 1u : (1u << p->start_depth);
     pl.roots = 0;
     return VC_OK;
+}
+
+// The launch shape, with the bitset search unless `nodes`; without it, too, where
+// its contexts (about 19 KB of memory per worker) are what does not fit.
+vc_status plan_launch(vc_ctx *ctx, uint32_t nmax, uint32_t depth, const vc_params *p, Plan &pl, bool serve,
+                      bool off16_ok = false, size_t mem_budget = 0, uint32_t adj_entries = 0, bool nodes = false)
+{
+    const vc_status st = plan_shape(ctx, nmax, depth, p, pl, serve, off16_ok, mem_budget, adj_entries, nodes);
+    if (st != VC_ENOMEM || nodes) return st;
+    return plan_shape(ctx, nmax, depth, p, pl, serve, off16_ok, mem_budget, adj_entries, true);
 }
 
 // A node budget limits a search by its number of nodes, and most of a budgeted

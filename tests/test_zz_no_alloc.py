@@ -118,3 +118,27 @@ def test_noalloc_refuses_what_does_not_fit(ctx):
     assert st == vcgpu.VC_ENOTSUP
     (r,), info, st = ctx.solve(small, vcgpu.Job(vcgpu.VC_MVC, 0, 2, 0), vcgpu.Params(), noalloc=True)
     assert st == vcgpu.VC_OK and r.solved and r.minimum == 2
+
+
+@pytest.mark.parametrize("n,budget,count", [(250, 1 << 12, 64), (400, 1 << 12, 64), (400, 0, 64), (2000, 1 << 12, 1), (2000, 0, 1)])
+def test_noalloc_takes_what_one_workgroup_fits(ctx, n, budget, count):
+    """The worklist follows the grid as it shrinks to the fixed scratch: sized
+    for the whole grid it alone took up to 208 MiB of the 128, and these sets
+    were refused."""
+    cases = [(n, graphgen.barabasi_albert(n, 3, 40 + i)) for i in range(min(count, 4))]
+    graphs = [vcgpu.csr_from_edges(n, e) for n, e in cases]
+    gs = ctx.upload([graphs[i % len(graphs)] for i in range(count)])
+    want = [_opt(n, e) for n, e in cases]
+    jobs = []
+    for i in range(count):
+        U, _ = vcgpu.upper_bound(graphs[i % len(graphs)], seed=3)
+        jobs.append(vcgpu.Job(vcgpu.VC_MVC, 0, U, budget))
+    got, info, st = ctx.solve(gs, jobs, vcgpu.Params(time_limit_ms=60000), raise_on_error=False, noalloc=True)
+    assert st in (vcgpu.VC_OK, vcgpu.VC_ETIMEOUT), st
+    assert info.list_size <= max(1024, 16 * info.workers)
+    for i, r in enumerate(got):
+        if r.solved or not budget:
+            assert r.solved and r.minimum == want[i % len(want)], (i, r.minimum)
+        if r.cover is not None:
+            og = O.from_edges(*cases[i % len(cases)])
+            assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == r.minimum
