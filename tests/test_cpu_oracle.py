@@ -82,7 +82,7 @@ def test_oracle_reproduces_reference_known_answers(name):
 def test_known_answer_files_match_reference_copies():
     """When the reference is mounted, the committed fixtures are exactly its files."""
     base = "/root/reference"
-    if not os.path.isdir(base):
+    if not os.path.isdir(base) or not os.listdir(base):
         pytest.skip("reference not mounted")
     for name, meta in KNOWN.items():
         g = load_reference_graph(os.path.join(base, meta["file"]), meta["index_base"])
