@@ -72,9 +72,13 @@ typedef struct {
 typedef struct {
     uint32_t version;           /* vc_version (-v) */
     uint32_t block_dim;         /* threads per workgroup (-b): a multiple of 64 up to 1024,
-                                   one search worker per 64-thread wave; 0 = auto.  When an
-                                   explicit workgroup's workers do not fit in LDS their node
-                                   state goes to HBM (as with -g 1) */
+                                   one search worker per 64-thread wave; 0 = auto (one worker
+                                   in an unbudgeted launch).  When an explicit workgroup's
+                                   workers do not fit in LDS with the bitset search's contexts
+                                   (7 or 16 KB each) their node state goes to HBM (as with
+                                   -g 1); with -g 0 it stays in LDS and the search runs
+                                   without contexts, up to the sizes that fit so (960 vertices
+                                   at 1,024 threads, 4,704 at 256, 19,840 at 64) */
     uint32_t num_blocks;        /* workgroups (-n); 0 = auto (one worker per SIMD; as many as
                                    fit when every graph has a node budget).  At most
                                    65535 workers (num_blocks x block_dim / 64) per launch.

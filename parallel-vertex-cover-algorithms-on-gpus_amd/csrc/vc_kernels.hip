@@ -2784,6 +2784,7 @@ struct vc_ctx {
     // until the last one stops (or the context is destroyed).
     std::mutex mem_mu;
     int active_servers = 0;
+    int wide_servers = 0;  // of those, the ones on more than half the CUs
     std::vector<std::pair<void *, bool>> deferred;  // (pointer, pinned host memory)
     std::vector<Block> spare;                       // blocks of freed sets (take_block)
 };
@@ -2899,7 +2900,7 @@ void *noalloc_scratch(int device)
 struct DispatchKey {
     int variant;
     uint32_t num_blocks, block_dim, version, start_depth, qsize, qthreshold, depth, want_covers;
-    uint32_t off16, adj, active0, roots, flush_share;  // kernel choice and staged start
+    uint32_t off16, adj, active0, roots, flush_share, bits_max;  // kernel choice, staged start, contexts
     size_t smem;
     uint64_t limit_ticks;
     const void *scratch;
@@ -3075,14 +3076,32 @@ void size_storage(Plan &pl, uint32_t nmax, uint32_t deg_bytes, bool off16 = fals
                  64u);
 }
 
-// LDS of a worker's contexts, and of a workgroup of wpb workers with their
-// node storage in LDS.
-uint32_t bits_lds(const Plan &pl) { return pl.bits_max == 0u ? 0u : pl.bits_max == vcg::kBitsMax ? vcg::kCtxLdsBytes : vcg::kCtxLdsSmall; }
-size_t lds_bytes(const Plan &pl, uint32_t wpb) { return (size_t)wpb * (bits_lds(pl) + pl.worker_bytes); }
+// LDS of a worker's contexts.
+uint32_t bits_lds(uint32_t bits_max) { return bits_max == 0u ? 0u : bits_max == vcg::kBitsMax ? vcg::kCtxLdsBytes : vcg::kCtxLdsSmall; }
+
+// The largest contexts that fit beside wpb workers' node storage of node_bytes
+// each in `limit` bytes of LDS (0 = none do): of 256 vertices, or of 128 where
+// those do not fit or no graph is larger.
+uint32_t fit_contexts(uint32_t nmax, uint32_t wpb, size_t node_bytes, size_t limit)
+{
+    for (uint32_t m : {vcg::kBitsMax, vcg::kBitsMaxSmall}) {
+        if (m == vcg::kBitsMax && nmax <= vcg::kBitsMaxSmall) continue;
+        if (wpb * (node_bytes + bits_lds(m)) <= limit) return m;
+    }
+    return 0u;
+}
 
 // Launch shape shared by the batch solve and the server: node storage,
 // workgroup, grid from the occupancy query, worklist, and the memory plan.
+// A server is idle most of the time, and every idle wave polls the launch-wide
+// words.  Two workers per CU served the mixed request stream (1,000 requests/s)
+// faster than the occupancy grid (856 vs 554 graphs/s; small requests p50 0.26 vs
+// 4.3 ms, p99 5.8 vs 37 ms).  In workgroups of four (max_vertices up to about
+// 4,700) they also leave half the CUs free for other kernels, and larger ones
+// leave LDS on every CU (plan_shape): with the occupancy grid a vc_solve issued
+// beside a server waited for it.
 constexpr uint32_t kServeWorkersPerCU = 2;
+uint32_t serve_blocks(const vc_ctx *ctx, uint32_t wpb) { return std::max<uint32_t>(1u, kServeWorkersPerCU * (uint32_t)ctx->cu_count / wpb); }
 // One worker per SIMD: a bitset search is a chain of scalar and vector
 // instructions with next to no memory access, so one wave nearly fills its
 // SIMD's issue slots, and more workers only share the same subtrees in smaller
@@ -3113,21 +3132,45 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
     // -g 0 forbids it); int16 degrees while n < 32768 (VC_FLAG_WIDE forces
     // int32).
     const bool wide = nmax >= 32768u || (p->flags & VC_FLAG_WIDE) != 0u;
-    pl.nodes = nodes;
     pl.bits_max = nodes ? 0u : vcg::kBitsMax;
     size_storage(pl, nmax, wide ? 4u : 2u);
     uint32_t wpb = block_dim / vcg::kWave;
+    // An automatic workgroup with contexts is one worker: contexts and node
+    // storage of a second one can push the adjacency, or the workgroup, out of
+    // the LDS that is free (beside a server, say).  64 / 256 threads: four
+    // 3-regular graphs of n = 108..120 1.19 / 1.24 ms, three of n = 225..250
+    // with half of all edges 8.3 / 8.8, BA n = 4,000 0.85 / 1.47, 1,024 graphs
+    // 17.7 / 17.9.
+    if (!p->block_dim && !nodes && !serve) wpb = 1u;
     bool hbm = wide || p->use_global_memory == 1;
+    // LDS that contexts may fill.  A server that is on every CU leaves 40 KB,
+    // which a solve of graphs of some 500 vertices needs to run beside it.
+    size_t ctx_limit = lds_limit;
     if (!hbm) {
         if (!p->block_dim)
-            while (wpb > 1 && lds_bytes(pl, wpb) > lds_limit) wpb /= 2;
-        // an explicit workgroup whose workers fit with smaller contexts only
-        if (!nodes && lds_bytes(pl, wpb) > lds_limit) pl.bits_max = vcg::kBitsMaxSmall;
-        hbm = lds_bytes(pl, wpb) > lds_limit;
+            while (wpb > 1 && wpb * (size_t)pl.worker_bytes > lds_limit) wpb /= 2;
+        hbm = wpb * (size_t)pl.worker_bytes > lds_limit;
+    }
+    if (serve && (p->num_blocks ? p->num_blocks : serve_blocks(ctx, wpb)) > (uint32_t)ctx->cu_count / 2u) ctx_limit -= 40u * 1024u;
+    if (!hbm && !nodes) {
+        // Contexts that do not fit: a solve's nodes go to HBM with contexts
+        // beside them (an explicit 1,024-thread workgroup, HBM with contexts
+        // against LDS without: cop_hat300-3 24 / 249 ms, er n = 320, p = 0.3, 118
+        // / 683, but BA n = 800, m = 4, 284 / 86), unless the caller wants
+        // them in LDS; a server, whose requests may all have budgets, goes
+        // without contexts.
+        pl.bits_max = fit_contexts(nmax, wpb, pl.worker_bytes, ctx_limit);
+        if (!pl.bits_max && !serve && p->use_global_memory != 0) hbm = true;
     }
     if (hbm && p->use_global_memory == 0) return VC_ENOTSUP;
     pl.variant = wide ? kHbm32 : hbm ? kHbm16 : kLds16;
-    if (hbm) size_storage(pl, nmax, wide ? 4u : 2u, false, 0u, kCandCapLarge);
+    if (hbm) {
+        if (!nodes) pl.bits_max = fit_contexts(nmax, wpb, 0u, ctx_limit);
+        size_storage(pl, nmax, wide ? 4u : 2u, false, 0u, kCandCapLarge);
+    } else {
+        size_storage(pl, nmax, 2u);
+    }
+    nodes = pl.nodes = !pl.bits_max;
     // LDS copy of the current graph's offsets (batch launches whose graphs
     // all have 2m < 2^16; a server reuses graph slots for new requests)
     pl.off16 = 0u;
@@ -3135,7 +3178,7 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
     if (!serve && off16_ok && pl.variant == kLds16) {
         Plan t = pl;
         size_storage(t, nmax, 2u, true);
-        if (lds_bytes(t, wpb) <= lds_limit) {
+        if (wpb * (size_t)(t.worker_bytes + bits_lds(t.bits_max)) <= lds_limit) {
             pl = t;
             pl.off16 = 1u;
         }
@@ -3146,8 +3189,10 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
             size_storage(ta, nmax, 2u, true, adj_entries);
             uint32_t wa = wpb;
             if (!p->block_dim)
-                while (wa > 1 && lds_bytes(ta, wa) > lds_limit) wa /= 2;
-            if (lds_bytes(ta, wa) <= lds_limit) {
+                while (wa > 1 && wa * (size_t)(ta.worker_bytes + bits_lds(ta.bits_max)) > lds_limit) wa /= 2;
+            // smaller contexts where those leave no room for the adjacency
+            if (!nodes) ta.bits_max = fit_contexts(nmax, wa, ta.worker_bytes, lds_limit);
+            if ((nodes || ta.bits_max) && wa * (size_t)(ta.worker_bytes + bits_lds(ta.bits_max)) <= lds_limit) {
                 pl = ta;
                 pl.off16 = 1u;
                 pl.adj = 1u;
@@ -3157,9 +3202,8 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
     }
     pl.wpb = wpb;
     pl.block_dim = wpb * vcg::kWave;
-    if (hbm && !nodes) pl.bits_max = (size_t)wpb * vcg::kCtxLdsBytes <= lds_limit ? vcg::kBitsMax : vcg::kBitsMaxSmall;
     // (a staged start shares one word of LDS)
-    pl.smem = std::max<size_t>(16u, (size_t)pl.wpb * (bits_lds(pl) + (hbm ? 0u : pl.worker_bytes)));
+    pl.smem = std::max<size_t>(16u, (size_t)pl.wpb * (bits_lds(pl.bits_max) + (hbm ? 0u : pl.worker_bytes)));
     if (pl.smem > lds_limit) return VC_ENOTSUP;
 
     int bpc = 0;
@@ -3170,14 +3214,7 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
     pl.blocks_per_cu = (uint32_t)bpc;
     uint32_t auto_blocks = (uint32_t)bpc * (uint32_t)ctx->cu_count;
     if (serve) {
-        // A server is idle most of the time, and every idle wave polls the
-        // launch-wide words.  kServeWorkersPerCU workers per CU served the
-        // mixed request stream (1,000 requests/s) faster than the occupancy
-        // grid (856 vs 554 graphs/s; small requests p50 0.26 vs 4.3 ms, p99
-        // 5.8 vs 37 ms), and the CUs left free run other kernels -- with the
-        // occupancy grid a vc_solve issued beside a server waited for it.
-        auto_blocks = std::min<uint32_t>(
-            auto_blocks, std::max<uint32_t>(1u, kServeWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
+        auto_blocks = std::min<uint32_t>(auto_blocks, serve_blocks(ctx, pl.wpb));
     } else if (!nodes) {
         auto_blocks = std::min<uint32_t>(
             auto_blocks, std::max<uint32_t>(1u, kSolveWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
@@ -3316,7 +3353,7 @@ void fill_args(SolveArgs &a, const Plan &pl, char *base, uint32_t version, uint3
     a.ctx = base + pl.off_ctx;
     a.ctx_bytes = pl.ctx_bytes;
     a.bits_max = pl.bits_max;
-    a.bits_lds = bits_lds(pl);
+    a.bits_lds = bits_lds(pl.bits_max);
     a.worker_bytes = pl.worker_bytes;
     a.depth = pl.depth;
     a.qsize = pl.qsize;
@@ -3756,7 +3793,7 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
         // The solve is bracketed by events outside the graph.
         DispatchKey key;
         std::memset(&key, 0, sizeof(key));
-        key.variant = pl.variant | (int)(pl.nodes << 8);
+        key.variant = pl.variant;
         key.num_blocks = pl.num_blocks;
         key.block_dim = pl.block_dim;
         key.version = a.version;
@@ -3770,6 +3807,7 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
         key.active0 = a.active0;
         key.roots = a.roots;
         key.flush_share = a.flush_share;
+        key.bits_max = pl.bits_max;
         key.smem = pl.smem;
         key.limit_ticks = a.limit_ticks;
         key.scratch = ctx->scratch;
@@ -3841,8 +3879,14 @@ constexpr uint32_t kShrinkMinN = 1024;
 constexpr uint32_t kShrinkMinLeaves = 64;  // of 1024
 constexpr int kShrinkMaxGraphs = 64;
 
-static bool shrinks(const vc_graphs *set, const vc_params *params)
+static bool shrinks(vc_ctx *ctx, const vc_graphs *set, const vc_params *params)
 {
+    {
+        // its workgroup asks for up to 144 KB of LDS: a server on every CU
+        // would keep it waiting
+        std::lock_guard<std::mutex> lk(ctx->mem_mu);
+        if (ctx->wide_servers) return false;
+    }
     return set->nmax >= kShrinkMinN && set->leaf_share >= kShrinkMinLeaves && set->count <= kShrinkMaxGraphs &&
            !(params->flags & VC_FLAG_GRAPH);
 }
@@ -4014,7 +4058,7 @@ vc_status vc_solve(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, cons
     if (!ctx || !set_c || !jobs || !params || !results) return VC_EINVAL;
     vc_graphs *set = const_cast<vc_graphs *>(set_c);
     if (!hip_ok(hipSetDevice(ctx->device))) return VC_EDEVICE;
-    return shrinks(set, params) ? solve_shrunk(ctx, set, jobs, params, results, covers, info)
+    return shrinks(ctx, set, params) ? solve_shrunk(ctx, set, jobs, params, results, covers, info)
                                 : solve_set(ctx, set, jobs, params, results, covers, info);
 }
 
@@ -4257,6 +4301,7 @@ constexpr uint64_t kUnit = 64;
 struct vc_server {
     vc_ctx *ctx = nullptr;
     bool counted = false;  // included in ctx->active_servers
+    bool wide = false;     // ... and in ctx->wide_servers
     vc_server_config cfg{};
     Plan pl{};
     SolveArgs a{};
@@ -4434,6 +4479,7 @@ void server_free(vc_server *s)
     if (s->counted) {
         std::lock_guard<std::mutex> lk(ctx->mem_mu);
         --ctx->active_servers;
+        ctx->wide_servers -= s->wide;
     }
     ctx_release(ctx, s->scratch, false);
     ctx_release(ctx, s->d_desc, false);
@@ -4494,6 +4540,11 @@ vc_status vc_server_start(vc_ctx *ctx, const vc_server_config *cfg, vc_server **
     if (st != VC_OK) {
         server_free(s);
         return st;
+    }
+    if (s->pl.num_blocks > (uint32_t)ctx->cu_count / 2u) {
+        std::lock_guard<std::mutex> lk(ctx->mem_mu);
+        ++ctx->wide_servers;
+        s->wide = true;
     }
     s->ring_size = next_pow2(std::max<uint32_t>(2u * slots, 1024u));
     bool ok = hip_ok(hipStreamCreateWithFlags(&s->kstream, hipStreamNonBlocking)) &&
