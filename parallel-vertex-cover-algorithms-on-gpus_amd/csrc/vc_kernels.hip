@@ -2032,6 +2032,8 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     uint32_t moved = 0;
     uint32_t flush_every = kFlushEvery;  // see flush_interval
     uint32_t rnd = wid * 2654435761u;    // random state (next_random)
+    bool dry = false;                    // a run of pops without a branch, since then
+    uint64_t dry_since = 0;
 
     for (;;) {
         // a subtree for the bitset search: its live vertices (whole: a root's
@@ -2054,9 +2056,39 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     copy_state<NodeT>(w.base, stk + (size_t)ts * slot_bytes, a.npad, w.n);
                 moved += copy_bytes<NodeT>(w.n);
                 w.sync();
+                --top;
+                if (BITS && !SERVE && a.version == 1 && top >= bot) {
+                    // Entries are offered where a node branches (below).  Nodes
+                    // that all end at once never get there, and a stack of dear
+                    // ones was worked off alone: with nodes of milliseconds
+                    // (a right child in a dense graph removes a thousand
+                    // vertices) the workers waited for one of them, 1,460 ms
+                    // for n = 1,500 and nine tenths of all edges instead of 32.
+                    // So after a run of such pops has taken offer_ticks, it
+                    // offers here, one entry after the other while they are
+                    // wanted.  (Not in servers, where a hard request that
+                    // donates more keeps the next ones waiting: 2.4 instead of
+                    // 1.9 ms; nor in the 7-waves kernels of budgeted launches,
+                    // which have no registers left for it: a batched step took
+                    // 3.33 s instead of 2.82.)
+                    const uint64_t now = wall_clock64();
+                    if (!dry) {
+                        dry = true;
+                        dry_since = now;
+                    } else if (now - dry_since >= a.offer_ticks) {
+                        dry = false;
+                        while (top >= bot && wants_donation(a, ld_rlx(&a.glob->counter), rnd) != 0u) {
+                            const uint32_t bs = (uint32_t)bot % a.depth;
+                            const uint2 mb = stk_meta[bs];
+                            if (uni(try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(mb.x), uni(mb.y), slot_bytes)) == 0u) break;
+                            ++bot;
+                            ++donations;
+                            moved += 2u * copy_bytes<NodeT>(w.n);
+                        }
+                    }
+                }
                 d = uni(m.x);
                 uint32_t v = uni(m.y);
-                --top;
                 cands_reset(c, false);
                 d += take_neighbours(w, v, c);
                 have = true;
@@ -2279,6 +2311,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         // then goes from the node storage straight to the worklist (a
         // BA n = 2,000 search, a chain of nodes that each donate their
         // right child, took 0.93 ms with the copy through the stack).
+        dry = false;
         const bool donate = a.version == 1 && wants_donation(a, ld_rlx(&a.glob->counter), rnd) != 0u;
         if (donate && top < bot && uni(try_enqueue(a, w, w.base, g, d, v, slot_bytes)) != 0u) {
             ++donations;
@@ -3335,8 +3368,10 @@ vc_status make_plan(vc_ctx *ctx, const vc_graphs *set, const vc_job *jobs, const
 }
 
 // Fills the launch arguments that depend only on the plan and the scratch base.
-void fill_args(SolveArgs &a, const Plan &pl, char *base, uint32_t version, uint32_t start_depth, uint64_t limit_ticks)
+void fill_args(SolveArgs &a, const vc_ctx *ctx, const Plan &pl, char *base, uint32_t version, uint32_t start_depth,
+               uint64_t limit_ticks)
 {
+    a.offer_ticks = (uint64_t)ctx->wall_khz / 5u;  // 200 us
     a.off16 = pl.off16;
     a.glob = reinterpret_cast<Global *>(base + pl.off_glob);
     a.stk = base + pl.off_stk;
@@ -3682,7 +3717,7 @@ SolveArgs solve_args(const vc_ctx *ctx, const vc_graphs *set, const vc_params *p
     a.num_graphs = (uint32_t)set->count;
     // deadline on the device wall clock (every wait loop checks it)
     const uint64_t ms = params->time_limit_ms ? params->time_limit_ms : 3600ull * 1000ull;
-    fill_args(a, pl, base, params->version, params->start_depth, ms * (uint64_t)ctx->wall_khz);
+    fill_args(a, ctx, pl, base, params->version, params->start_depth, ms * (uint64_t)ctx->wall_khz);
     a.flush_share = std::max<uint32_t>(1u, pl.workers / std::max<uint32_t>(1u, a.num_graphs));
     // staged start (vcg::dormant_join) when the grid is automatic and the
     // roots could keep fewer than half the workers busy; the adjacency
@@ -4574,7 +4609,7 @@ vc_status vc_server_start(vc_ctx *ctx, const vc_server_config *cfg, vc_server **
     a.gstate = s->d_state;
     a.num_graphs = 0;  // slot state is set by the worker that claims a request
     const uint64_t ms = cfg->time_limit_ms ? cfg->time_limit_ms : 3600ull * 1000ull;
-    fill_args(a, s->pl, static_cast<char *>(s->scratch), VC_HYBRID, 0u, ms * (uint64_t)ctx->wall_khz);
+    fill_args(a, ctx, s->pl, static_cast<char *>(s->scratch), VC_HYBRID, 0u, ms * (uint64_t)ctx->wall_khz);
     a.serving = 1;
     a.ring_mask = s->ring_size - 1u;
     a.req_ring = s->h_ring;
