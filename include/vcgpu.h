@@ -170,7 +170,9 @@ vc_status vc_graphs_free(vc_ctx *ctx, vc_graphs *set);
 
 /* Solve every graph of the set in ONE persistent launch: jobs[count],
  * results[count]; covers == NULL or covers[i] == NULL skips that cover,
- * otherwise covers[i] receives vertexNum bytes (1 = in cover).
+ * otherwise covers[i] receives vertexNum bytes (1 = in cover).  (Two launches,
+ * one after the other in the call's time limit, when some jobs have node budgets,
+ * of 2^15 nodes in all or more, and others have none.)
  * Replaces src/main.cu:219-366 (stacks, worklist, launch, readback) for the
  * four kernels GlobalWorkList{,Parameterized}_{shared,global}_kernel
  * (src/GlobalWorkList.cuh:12-18, src/GlobalWorkListParameterized.cuh:12-18) and

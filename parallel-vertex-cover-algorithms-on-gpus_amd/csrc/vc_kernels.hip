@@ -2942,8 +2942,10 @@ struct DispatchKey {
 
 struct vc_graphs {
     int count = 0;
+    int capacity = 0;             // graphs that its buffers have room for
     vc_graphs *rest = nullptr;    // what shrink_kernel leaves of the set (buffers kept across solves)
-    bool borrowed = false;        // d_words belongs to the context
+    vc_graphs *part[2] = {};      // its graphs with and without a budget (solve_parts; likewise)
+    bool borrowed = false;        // d_words belongs to the context or another set
     int device = 0;
     Block dev;                    // d_words, d_desc, d_covers and d_state
     Block pinned;                 // h_state, h_glob and h_cov
@@ -2984,10 +2986,11 @@ inline size_t block_up(size_t bytes) { return (bytes + 255u) / 256u * 256u; }
 // context's), descriptors, cover bitmaps and graph states.
 bool take_device(vc_ctx *ctx, vc_graphs *s, size_t words)
 {
-    const size_t csr = block_up(sizeof(uint32_t) * words), desc = block_up(sizeof(GDesc) * (size_t)s->count);
+    s->capacity = s->count;
+    const size_t csr = block_up(sizeof(uint32_t) * words), desc = block_up(sizeof(GDesc) * (size_t)s->capacity);
     const size_t cov = block_up(sizeof(uint32_t) * (size_t)s->cover_words);
     s->device = ctx->device;
-    if (!take_block(ctx, csr + desc + cov + sizeof(GState) * (size_t)s->count, false, s->dev)) return false;
+    if (!take_block(ctx, csr + desc + cov + sizeof(GState) * (size_t)s->capacity, false, s->dev)) return false;
     if (words) s->d_words = reinterpret_cast<uint32_t *>(s->dev.p);
     s->d_desc = reinterpret_cast<GDesc *>(s->dev.p + csr);
     s->d_covers = reinterpret_cast<uint32_t *>(s->dev.p + csr + desc);
@@ -3142,6 +3145,7 @@ uint32_t serve_blocks(const vc_ctx *ctx, uint32_t wpb) { return std::max<uint32_
 // workers, 17.2 with 512, 26 with 1,792).
 constexpr uint32_t kSolveWorkersPerCU = 4;
 constexpr uint32_t kMaxBlockDim = 1024;   // the solve kernels' launch bound
+constexpr uint32_t kDefaultLimitMs = 3600u * 1000u;  // a launch's time limit when none is given
 constexpr uint32_t kMaxWorkers = 0xFFFFu; // 16-bit worker counts in the termination word
 
 vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_params *p, Plan &pl, bool serve,
@@ -3628,6 +3632,8 @@ vc_status vc_graphs_free(vc_ctx *ctx, vc_graphs *s)
     if (!s) return VC_EINVAL;
     if (ctx) (void)hipSetDevice(ctx->device);
     if (s->rest) vc_graphs_free(ctx, s->rest);
+    for (vc_graphs *p : s->part)
+        if (p) vc_graphs_free(ctx, p);
     if (s->exec) (void)hipGraphExecDestroy(s->exec);
     if (s->graph) (void)hipGraphDestroy(s->graph);
     ctx_release(ctx, s->h_shrink, true);
@@ -3716,7 +3722,7 @@ SolveArgs solve_args(const vc_ctx *ctx, const vc_graphs *set, const vc_params *p
     a.covers = set->d_covers;
     a.num_graphs = (uint32_t)set->count;
     // deadline on the device wall clock (every wait loop checks it)
-    const uint64_t ms = params->time_limit_ms ? params->time_limit_ms : 3600ull * 1000ull;
+    const uint64_t ms = params->time_limit_ms ? params->time_limit_ms : kDefaultLimitMs;
     fill_args(a, ctx, pl, base, params->version, params->start_depth, ms * (uint64_t)ctx->wall_khz);
     a.flush_share = std::max<uint32_t>(1u, pl.workers / std::max<uint32_t>(1u, a.num_graphs));
     // staged start (vcg::dormant_join) when the grid is automatic and the
@@ -3781,7 +3787,7 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
         for (int i = 0; i < set->count; ++i) want_covers |= covers[i] != nullptr;
     // readback buffers, pinned and mapped: publish_kernel writes them
     if (!set->h_state) {
-        const size_t state = block_up(sizeof(GState) * (size_t)set->count), glob = block_up(sizeof(Global));
+        const size_t state = block_up(sizeof(GState) * (size_t)set->capacity), glob = block_up(sizeof(Global));
         if (!take_block(ctx, state + glob + sizeof(uint32_t) * (size_t)set->cover_words, true, set->pinned)) return VC_ENOMEM;
         set->h_state = reinterpret_cast<GState *>(set->pinned.p);
         set->h_glob = reinterpret_cast<Global *>(set->pinned.p + state);
@@ -3903,6 +3909,91 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
         }
     }
     fill_info(info, ctx, pl, ms, total_nodes, idle, donations, steals, hg.t0, last_exit, hg.state_bytes);
+    return overall;
+}
+
+// vc_solve of a set in which some graphs have a budget and others have not: one
+// launch each, first the graphs with one (searches_nodes), in the time that the
+// call has.  In one launch the budgets' general search had four workers per CU
+// instead of 28: 4,095 graphs at 2^20 nodes and one without a budget took 14.4
+// s, in two launches 2.84.  Budgets of fewer than kSplitNodes nodes in all cost
+// less in one launch (about 5 ns more a node) than a second launch does.
+constexpr uint64_t kSplitNodes = 1u << 15;
+
+static vc_status solve_parts(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, const vc_params *params, vc_result *results,
+                             uint8_t *const *covers, vc_launch_info *info)
+{
+    uint64_t nodes = 0;
+    int with = 0;
+    for (int i = 0; i < set->count; ++i) {
+        with += jobs[i].max_nodes != 0u;
+        nodes += std::min(jobs[i].max_nodes, kSplitNodes);
+    }
+    if (with == 0 || with == set->count || nodes < kSplitNodes) return solve_set(ctx, set, jobs, params, results, covers, info);
+    for (int i = 0; i < set->count; ++i)
+        if ((!set->borrowed && jobs[i].upper_bound > set->h_desc[i].n) || (jobs[i].instance != VC_MVC && jobs[i].instance != VC_PVC))
+            return VC_EINVAL;
+    vc_status overall = VC_OK;
+    vc_params p = *params;
+    vc_launch_info sum;
+    for (int half = 0; half < 2; ++half) {
+        vc_graphs *s = set->part[half];
+        if (!s) {
+            s = new vc_graphs();
+            s->count = set->count;
+            s->borrowed = true;
+            s->cover_words = set->cover_words;
+            if (!take_device(ctx, s, 0)) {
+                vc_graphs_free(ctx, s);
+                return VC_ENOMEM;
+            }
+            set->part[half] = s;
+        }
+        std::vector<int> at;
+        std::vector<vc_job> part_jobs;
+        std::vector<uint8_t *> part_covers;
+        s->h_desc.clear();
+        s->nmax = 0;
+        for (int i = 0; i < set->count; ++i) {
+            if ((jobs[i].max_nodes != 0u) != (half == 0)) continue;
+            at.push_back(i);
+            part_jobs.push_back(jobs[i]);
+            part_covers.push_back(covers ? covers[i] : nullptr);
+            s->h_desc.push_back(set->h_desc[i]);
+            s->nmax = std::max(s->nmax, set->h_desc[i].n);
+        }
+        s->count = (int)at.size();
+        s->d_words = set->d_words;
+        s->dirty = true;
+        std::vector<vc_result> part_results(at.size());
+        vc_launch_info one;
+        const vc_status st = solve_set(ctx, s, part_jobs.data(), &p, part_results.data(), part_covers.data(), &one);
+        if (st != VC_OK && st != VC_ETIMEOUT) return st;
+        if (st != VC_OK) overall = st;
+        const uint32_t before_us = half ? (uint32_t)(sum.active_ms * 1000.f) : 0u;
+        for (size_t i = 0; i < at.size(); ++i) {
+            results[at[i]] = part_results[i];
+            if (results[at[i]].done_us) results[at[i]].done_us += before_us;
+        }
+        if (half == 0) {
+            sum = one;
+            const uint32_t limit = params->time_limit_ms ? params->time_limit_ms : kDefaultLimitMs;
+            p.time_limit_ms = limit > one.kernel_ms + 1.f ? limit - (uint32_t)one.kernel_ms : 1u;
+        } else {
+            // the launch shape is that of the larger part
+            const vc_launch_info &big = 2 * with >= set->count ? sum : one;
+            vc_launch_info all = big;
+            const double span0 = (double)sum.kernel_ms * sum.workers, span1 = (double)one.kernel_ms * one.workers;
+            all.idle_fraction = span0 + span1 > 0 ? (float)((sum.idle_fraction * span0 + one.idle_fraction * span1) / (span0 + span1)) : 0.f;
+            all.kernel_ms = sum.kernel_ms + one.kernel_ms;
+            all.active_ms = sum.active_ms + one.active_ms;
+            all.tree_nodes = sum.tree_nodes + one.tree_nodes;
+            all.donations = sum.donations + one.donations;
+            all.steals = sum.steals + one.steals;
+            all.state_bytes = sum.state_bytes + one.state_bytes;
+            if (info) *info = all;
+        }
+    }
     return overall;
 }
 
@@ -4054,7 +4145,7 @@ static vc_status solve_shrunk(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, c
                 rest_covers[i] = rest_bytes[i].data();
             }
         }
-        overall = solve_set(ctx, rest, rest_jobs.data(), params, rest_results.data(), want_covers ? rest_covers.data() : nullptr, info);
+        overall = solve_parts(ctx, rest, rest_jobs.data(), params, rest_results.data(), want_covers ? rest_covers.data() : nullptr, info);
         if (overall != VC_OK && overall != VC_ETIMEOUT) return overall;
         float ms = 0.f;
         if (info && hipEventElapsedTime(&ms, began, ctx->ev1) == hipSuccess) info->kernel_ms = ms;
@@ -4094,7 +4185,7 @@ vc_status vc_solve(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, cons
     vc_graphs *set = const_cast<vc_graphs *>(set_c);
     if (!hip_ok(hipSetDevice(ctx->device))) return VC_EDEVICE;
     return shrinks(ctx, set, params) ? solve_shrunk(ctx, set, jobs, params, results, covers, info)
-                                : solve_set(ctx, set, jobs, params, results, covers, info);
+                                     : solve_parts(ctx, set, jobs, params, results, covers, info);
 }
 
 vc_status vc_solve_noalloc(vc_ctx *ctx, const vc_graphs *set_c, const vc_job *jobs, const vc_params *params,
@@ -4608,7 +4699,7 @@ vc_status vc_server_start(vc_ctx *ctx, const vc_server_config *cfg, vc_server **
     a.gdesc = s->d_desc;
     a.gstate = s->d_state;
     a.num_graphs = 0;  // slot state is set by the worker that claims a request
-    const uint64_t ms = cfg->time_limit_ms ? cfg->time_limit_ms : 3600ull * 1000ull;
+    const uint64_t ms = cfg->time_limit_ms ? cfg->time_limit_ms : kDefaultLimitMs;
     fill_args(a, ctx, s->pl, static_cast<char *>(s->scratch), VC_HYBRID, 0u, ms * (uint64_t)ctx->wall_khz);
     a.serving = 1;
     a.ring_mask = s->ring_size - 1u;
