@@ -1086,7 +1086,7 @@ __device__ __forceinline__ uint32_t bit_level(const SolveArgs &a, const BitsLds 
                     ++b.since;
                     if (a.version == 1u && b.top >= b.bot &&
                         (b.since >= kDonateEvery || b.top - b.bot + 1 >= (int)kDonateBatch)) {
-                        b.want = wants_donation(a, counter_next, b.rnd);
+                        b.want = wants_donation<true>(a, counter_next, b.rnd);
                         if (b.want != 0u && uni((uint32_t)(state_next >> 32)) == 0u) return leave(kBitsDonate);
                     }
                 }

@@ -1386,14 +1386,17 @@ __device__ __forceinline__ uint32_t next_random(uint32_t &state)
 // shortage only about twice as many as items are missing act on it (returns how
 // many are missing, 0 = do not donate): when all
 // did, a search of 470,000 nodes on 4,096 workers made 183,000 donations and
-// took 48 ms, against 17 ms on 1,024 workers.
+// took 48 ms, against 17 ms on 1,024 workers.  (Without GATE, in launches of only
+// budgeted graphs, all of them act: 512 graphs at 2^20 nodes 513 instead of 535
+// ms.)
+template <bool GATE>
 __device__ __forceinline__ uint32_t wants_donation(const SolveArgs &a, unsigned long long counter, uint32_t &rnd)
 {
     const uint32_t lo = uni((uint32_t)counter), enq = (uint32_t)max((int)uni((uint32_t)(counter >> 32)), 0);
     const uint32_t waiting = lo & 0xFFFFu, busy = (lo >> 16) - waiting;
     if (waiting == 0u || enq >= waiting || enq >= a.qthreshold) return 0u;
     const uint32_t missing = min(waiting, a.qthreshold) - enq;
-    if (2u * missing >= busy) return missing;
+    if (!GATE || 2u * missing >= busy) return missing;
     return ((next_random(rnd) * busy) >> 16) < 2u * missing ? missing : 0u;
 }
 
@@ -1716,7 +1719,7 @@ struct Acquired {
 // Batch launches count their roots in the termination word's "enqueued"
 // field from the start (init_kernel), like items of the worklist, so
 // termination is simply waiting == registered with nothing enqueued.
-template <bool SERVE, class N>
+template <bool SERVE, bool GATE, class N>
 __device__ __forceinline__ Acquired acquire(const SolveArgs &a, const N &w, uint32_t slot_bytes, bool counted, uint32_t rnd)
 {
     Acquired r = {0u, kNone, 0u, kNone, 0u, kNone, 0u};
@@ -1733,11 +1736,11 @@ __device__ __forceinline__ Acquired acquire(const SolveArgs &a, const N &w, uint
         // One poll is one read of the termination word: items (batch: and
         // roots) are there only when its "enqueued" field says so, and with
         // fewer items than waiting workers only about twice as many workers
-        // as items try to take one.
+        // as items try to take one (GATE, see wants_donation).
         const unsigned long long seen = ld_rlx(&a.glob->counter);
         const uint32_t lo = uni((uint32_t)seen), hi = uni((uint32_t)(seen >> 32));
         const uint32_t waiting = lo & 0xFFFFu, reg = lo >> 16;
-        if ((int)hi > 0 && (2u * hi >= waiting || ((next_random(rnd) * waiting) >> 16) < 2u * hi)) {
+        if ((int)hi > 0 && (!GATE || 2u * hi >= waiting || ((next_random(rnd) * waiting) >> 16) < 2u * hi)) {
             // Take one off "enqueued" and leave "waiting" in one step; with
             // nothing there (the field was 0 or, while others are at this
             // point, below) put both back.  What was taken stands for
@@ -2077,7 +2080,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                         dry_since = now;
                     } else if (now - dry_since >= a.offer_ticks) {
                         dry = false;
-                        while (top >= bot && wants_donation(a, ld_rlx(&a.glob->counter), rnd) != 0u) {
+                        while (top >= bot && wants_donation<BITS>(a, ld_rlx(&a.glob->counter), rnd) != 0u) {
                             const uint32_t bs = (uint32_t)bot % a.depth;
                             const uint2 mb = stk_meta[bs];
                             if (uni(try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(mb.x), uni(mb.y), slot_bytes)) == 0u) break;
@@ -2101,7 +2104,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 }
                 if (lane_id() == 0 && ld_rlx(&a.glob->cancel)) st_rlx(&a.glob->done_flag, 1u);
                 const uint64_t t_idle = wall_clock64();
-                Acquired q = acquire<SERVE>(a, w, slot_bytes, counted, rnd ^ (uint32_t)t_idle);
+                Acquired q = acquire<SERVE, BITS>(a, w, slot_bytes, counted, rnd ^ (uint32_t)t_idle);
                 counted = false;
                 idle_ticks += wall_clock64() - t_idle;
                 if (q.kind == 0) break;
@@ -2312,7 +2315,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         // BA n = 2,000 search, a chain of nodes that each donate their
         // right child, took 0.93 ms with the copy through the stack).
         dry = false;
-        const bool donate = a.version == 1 && wants_donation(a, ld_rlx(&a.glob->counter), rnd) != 0u;
+        const bool donate = a.version == 1 && wants_donation<BITS>(a, ld_rlx(&a.glob->counter), rnd) != 0u;
         if (donate && top < bot && uni(try_enqueue(a, w, w.base, g, d, v, slot_bytes)) != 0u) {
             ++donations;
             moved += copy_bytes<NodeT>(w.n);
