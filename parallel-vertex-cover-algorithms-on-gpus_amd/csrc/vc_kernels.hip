@@ -2822,7 +2822,7 @@ struct vc_ctx {
     int active_servers = 0;
     int wide_servers = 0;  // of those, the ones on more than half the CUs
     std::vector<std::pair<void *, bool>> deferred;  // (pointer, pinned host memory)
-    std::vector<Block> spare;                       // blocks of freed sets (take_block)
+    std::vector<Block> spare;                       // blocks of freed sets, oldest first (take_block)
 };
 
 void free_now(void *p, bool host)
@@ -2852,8 +2852,10 @@ void ctx_release(vc_ctx *ctx, void *p, bool host)
 // other uploads, solves and frees a set per question, and allocating and
 // freeing its eight buffers was half of such a call (four graphs of n = 36..40:
 // 1.12 ms with them, 0.53 now).  A spare block is never in use: a solve
-// returns after its last kernel.  At most kSpareBlocks of kSpareBytes each are
-// kept, until the context is destroyed; larger ones are freed with their set.
+// returns after its last kernel.  The last kSpareBlocks of up to kSpareBytes each
+// are kept, until the context is destroyed; larger ones are freed with their set.
+// (When the first ones stayed, a program that had freed eight blocks of other
+// sizes before had none of this: 0.226 instead of 0.166 ms a question.)
 constexpr size_t kSpareBytes = 1u << 20;
 constexpr size_t kSpareBlocks = 8;
 bool take_block(vc_ctx *ctx, size_t bytes, bool host, Block &out)
@@ -2863,11 +2865,10 @@ bool take_block(vc_ctx *ctx, size_t bytes, bool host, Block &out)
     size = std::max(size, bytes);
     if (size <= kSpareBytes) {
         std::lock_guard<std::mutex> lk(ctx->mem_mu);
-        for (Block &b : ctx->spare)
-            if (b.host == host && b.bytes == size) {
-                out = b;
-                b = ctx->spare.back();
-                ctx->spare.pop_back();
+        for (auto b = ctx->spare.begin(); b != ctx->spare.end(); ++b)
+            if (b->host == host && b->bytes == size) {
+                out = *b;
+                ctx->spare.erase(b);
                 return true;
             }
     }
@@ -2878,18 +2879,19 @@ bool take_block(vc_ctx *ctx, size_t bytes, bool host, Block &out)
     return true;
 }
 
-// Keeps b (of a set on `device`) for a later set, or frees it.
+// Keeps b (of a set on `device`) for a later set, in place of the oldest spare
+// one if there are enough, or frees it.
 void give_block(vc_ctx *ctx, int device, Block &b)
 {
-    const Block x = b;
+    Block x = b;
     b = Block{};
     if (!x.p) return;
     if (ctx && ctx->device == device && x.bytes <= kSpareBytes) {
         std::lock_guard<std::mutex> lk(ctx->mem_mu);
-        if (ctx->spare.size() < kSpareBlocks) {
-            ctx->spare.push_back(x);
-            return;
-        }
+        ctx->spare.push_back(x);
+        if (ctx->spare.size() <= kSpareBlocks) return;
+        x = ctx->spare.front();
+        ctx->spare.erase(ctx->spare.begin());
     }
     ctx_release(ctx, x.p, x.host);
 }
