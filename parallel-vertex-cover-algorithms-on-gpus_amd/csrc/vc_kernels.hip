@@ -4282,7 +4282,7 @@ extern "C" vc_status vc_autotune(vc_ctx *ctx, const vc_graphs *set, const vc_job
     // shape ends early instead of running the whole sample.
     std::vector<vc_params> cands;
     // The automatic workgroup goes first, and another shape has to be 5% faster
-    // than the best before it: on a sample shapes differ by less than two runs of
+    // than the best before it, twice: on a sample shapes differ by less than two runs of
     // one do (512 graphs at 2^20 nodes: 64, 128 and 256 threads 505-550 ms), and
     // one picked for that can be 7% slower on the whole (4,096 graphs, 64
     // threads: 3.04 s, 256: 2.82).
@@ -4325,18 +4325,28 @@ extern "C" vc_status vc_autotune(vc_ctx *ctx, const vc_graphs *set, const vc_job
             if (!cands[i].time_limit_ms || cap < cands[i].time_limit_ms) cands[i].time_limit_ms = cap;
         }
         vc_launch_info info;
-        vc_status st = vc_solve(ctx, set, jobs, &cands[i], res.data(), nullptr, &info);
-        if (st != VC_OK && st != VC_ETIMEOUT) continue;
         // time per solved graph, so a shape that finishes more graphs within
-        // the jobs' node budgets is not penalised for it
-        uint32_t solved = 0;
-        for (const vc_result &r : res) solved += r.solved;
-        const float t = info.kernel_ms / (float)std::max<uint32_t>(solved, 1u);
-        if (best_i < 0 || t < 0.95f * best_t) {
-            best_t = t;
-            best_kernel_ms = info.kernel_ms;
-            best_i = (int)i;
+        // the jobs' node budgets is not penalised for it; 0 = it does not run
+        auto time = [&](vc_params &p) -> float {
+            const vc_status st = vc_solve(ctx, set, jobs, &p, res.data(), nullptr, &info);
+            if (st != VC_OK && st != VC_ETIMEOUT) return 0.f;
+            uint32_t solved = 0;
+            for (const vc_result &r : res) solved += r.solved;
+            return info.kernel_ms / (float)std::max<uint32_t>(solved, 1u);
+        };
+        float t = time(cands[i]);
+        if (t <= 0.f || (best_i >= 0 && t >= 0.95f * best_t)) continue;
+        if (best_i >= 0) {
+            // once more, the best one first: it may have had a slow run
+            const float again = time(cands[(size_t)best_i]);
+            if (again > 0.f) best_t = std::min(best_t, again);
+            if (t >= 0.95f * best_t) continue;
+            t = time(cands[i]);
+            if (t <= 0.f || t >= 0.95f * best_t) continue;
         }
+        best_t = t;
+        best_kernel_ms = info.kernel_ms;
+        best_i = (int)i;
     }
     if (best_i < 0) return VC_ENOTSUP;
     *best = cands[best_i];
