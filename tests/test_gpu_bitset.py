@@ -3,6 +3,8 @@ at the sizes where its layout changes: one vertex below, at and above each
 context size (32, 48, 64, 96, 128 and 256 vertices; 64 K vertices fill K slots
 of a lane).  MVC, and PVC at k = MVC - 1 and MVC, against the CPU oracle; every
 cover is checked.  All answers are whole numbers: no tolerance."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -16,7 +18,8 @@ SIZES = [s + d for s in (32, 48, 64, 96, 128, 256) for d in (-1, 0, 1)]
 
 
 def _graphs(n):
-    # no vertex of degree 0 to 2 at the root, so the first context has n vertices
+    # dense: no vertex of degree 0 to 2 at the root, so the first context has n
+    # vertices; sparse: about a sixteenth of them have, and reductions come first
     out = [("dense", graphgen.erdos_renyi(n, 0.9, 4000 + n))]
     if n <= 97:
         out.append(("sparse", graphgen.erdos_renyi(n, 6.0 / n, 5000 + n)))
@@ -105,3 +108,71 @@ def test_dear_nodes_that_end_at_once_are_shared(ctx):
                 assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == r.minimum
     assert len(minima) == 1, minima
     assert ms["default"] < 5.0 * ms["every worker"], ms
+
+
+@functools.lru_cache(maxsize=None)
+def _regular3(n):
+    e = graphgen.regular3_rewired(n, 11)
+    want, stats, _ = O.mvc(O.from_edges(n, e), max_nodes=2_000_000)
+    assert stats["completed"]
+    return e, want
+
+
+def _sparse_core(n):
+    """n vertices of degree 3 and 4 (nothing to reduce), and its MVC: 3-regular
+    graphs of at most 128 vertices (one of up to 194), and for odd n a K5."""
+    parts, at, want = [], 0, 0
+    left = n
+    if n % 2:
+        parts.append(np.array([(i, j) for i in range(5) for j in range(i + 1, 5)], np.uint32))
+        at, want, left = 5, 4, n - 5
+    for size in [left] if left <= 194 else [128, left - 128]:
+        e, m = _regular3(size)
+        parts.append(np.asarray(e, np.uint32) + np.uint32(at))
+        at, want = at + size, want + m
+    return np.concatenate(parts), want
+
+
+def _solve_three(ctx, n, e, want, params):
+    """MVC, and PVC on both sides of it, on a graph whose MVC is known."""
+    og = O.from_edges(n, e)
+    gs = ctx.upload([vcgpu.csr_from_edges(n, e)] * 3)
+    jobs = [vcgpu.Job(vcgpu.VC_MVC, 0, n - 1, 0), vcgpu.Job(vcgpu.VC_PVC, want - 1, n - 1, 0), vcgpu.Job(vcgpu.VC_PVC, want, n - 1, 0)]
+    (mvc, no, yes), _, st = ctx.solve(gs, jobs, params)
+    assert st == vcgpu.VC_OK
+    assert mvc.solved and mvc.minimum == want, (n, mvc.minimum, want)
+    assert no.solved and not no.k_found, n
+    assert yes.solved and yes.k_found, n
+    for r in (mvc, yes):
+        assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == want, n
+
+
+@pytest.mark.parametrize("n", [127, 128, 129, 160, 191, 192, 194, 254, 255, 256, 257])
+def test_sparse_remainders_of_four_slots_match_oracle(ctx, n):
+    """The rounds of the clique cover over all lanes, where vertex ids fill a byte:
+    nothing is reduced at the root, so the first context has n vertices."""
+    e, want = _sparse_core(n)
+    _solve_three(ctx, n, e, want, vcgpu.Params(time_limit_ms=60000))
+
+
+@pytest.mark.parametrize("version", [vcgpu.VC_HYBRID, vcgpu.VC_STACK_ONLY])
+@pytest.mark.parametrize("core", SIZES)
+def test_remainders_of_larger_graphs_match_oracle(ctx, core, version):
+    """Graphs of more than 256 vertices whose reduced root has exactly `core`: every
+    third core vertex carries pendant paths of two, which the leaf rule takes off
+    again (one cover vertex each).  Here the contexts are made from node state."""
+    cores = [graphgen.erdos_renyi(core, 0.9, 4000 + core)]
+    wants = [O.mvc(O.from_edges(core, cores[0]), max_nodes=2_000_000)[0]]
+    if core >= 48 and (core < 200 or version == vcgpu.VC_HYBRID):  # (seconds on the four static paths)
+        e, m = _sparse_core(core)
+        cores.append(e)
+        wants.append(m)
+    pairs = (300 - core) // 2 if core < 200 else 60
+    n = core + 2 * pairs
+    # ids mixed: core vertex i is vertex keep[i]
+    ids = np.random.default_rng(core).permutation(n).astype(np.uint32)
+    keep, rest = np.sort(ids[:core]), ids[core:]
+    for e, want in zip(cores, wants):
+        hang = [(keep[(3 * i) % core], rest[2 * i]) for i in range(pairs)] + [(rest[2 * i], rest[2 * i + 1]) for i in range(pairs)]
+        full = np.concatenate([keep[np.asarray(e, np.int64)], np.asarray(hang, np.uint32)]).astype(np.uint32)
+        _solve_three(ctx, n, full, want + pairs, vcgpu.Params(version=version, start_depth=2, time_limit_ms=60000))
