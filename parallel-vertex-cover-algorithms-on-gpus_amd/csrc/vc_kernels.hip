@@ -3197,8 +3197,8 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
     if (!hbm && !nodes) {
         // Contexts that do not fit: a solve's nodes go to HBM with contexts
         // beside them (an explicit 1,024-thread workgroup, HBM with contexts
-        // against LDS without: cop_hat300-3 24 / 249 ms, er n = 320, p = 0.3, 118
-        // / 683, but BA n = 800, m = 4, 284 / 86), unless the caller wants
+        // against LDS without: cop_hat300-3 26 / 234 ms, er n = 320, p = 0.3, 107
+        // / 675, but BA n = 800, m = 4, 158 / 87), unless the caller wants
         // them in LDS; a server, whose requests may all have budgets, goes
         // without contexts.
         pl.bits_max = fit_contexts(nmax, wpb, pl.worker_bytes, ctx_limit);
@@ -3258,8 +3258,12 @@ vc_status plan_shape(vc_ctx *ctx, uint32_t nmax_in, uint32_t depth, const vc_par
     if (serve) {
         auto_blocks = std::min<uint32_t>(auto_blocks, serve_blocks(ctx, pl.wpb));
     } else if (!nodes) {
-        auto_blocks = std::min<uint32_t>(
-            auto_blocks, std::max<uint32_t>(1u, kSolveWorkersPerCU * (uint32_t)ctx->cu_count / pl.wpb));
+        // HBM nodes with 128-vertex contexts (an explicit large workgroup): more
+        // of the search is the general one, which waits for memory.  1,024
+        // threads, 4 / 8 / 16 workers per CU: BA n = 800, m = 4, 284 / 158 / 120
+        // ms, er n = 320, p = 0.3, 123 / 107 / 152, cop_hat300-3 24 / 26 / 36.
+        const uint32_t per_cu = hbm && pl.bits_max == vcg::kBitsMaxSmall ? 2u * kSolveWorkersPerCU : kSolveWorkersPerCU;
+        auto_blocks = std::min<uint32_t>(auto_blocks, std::max<uint32_t>(1u, per_cu * (uint32_t)ctx->cu_count / pl.wpb));
     }
     pl.num_blocks = p->num_blocks ? p->num_blocks : auto_blocks;
     // the termination word counts waiting and registered workers in 16-bit
