@@ -2029,6 +2029,17 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
     Cands c;            // rule candidates listed since the last passes
     uint32_t off16_g = kNone;  // graph whose offsets the LDS copy holds
     uint64_t pending = 0, total_nodes = 0, idle_ticks = 0, donations = 0, steals = 0;
+    // The worker's statistics: in registers, or, in the kernels of budgeted
+    // launches, whose 72 VGPRs they would take part in spilling, added to its
+    // record in memory at once.
+    constexpr bool kTally = !BITS && !SERVE;
+    auto tally = [&](uint64_t &count, uint64_t WorkerStats::*field, uint64_t x) {
+        if constexpr (kTally) {
+            if (lane_id() == 0) a.wstats[wid].*field += x;
+        } else {
+            count += x;
+        }
+    };
     // HBM bytes of the node state moved since the last flush: stack pushes
     // and pops, steals (ring slot in) and donations (stack slot to ring slot,
     // two); flush_nodes adds them to the launch total
@@ -2043,6 +2054,22 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         // graph as it is), or a donated one
         uint32_t bits = 0, bits_ctx = kNone, bits_word = 0;
         bool whole = false;
+        // Every control value of the loop is wave-uniform, but the compiler loses
+        // sight of that where values meet behind a branch on the lane number,
+        // and then carries them in VGPRs, under exec masks: the 7-waves kernel
+        // spilled 43 of them, a kilobyte of writes per node (none with these
+        // lines).
+        if constexpr (!BITS) {
+            top = (int)uni((uint32_t)top);
+            bot = (int)uni((uint32_t)bot);
+            d = uni(d);
+            g = uni(g);
+            have = uni(have) != 0u;
+            descend = uni(descend);
+            pending = uni64(pending);
+            moved = uni(moved);
+            flush_every = uni(flush_every);
+        }
         if (!have) {
             if (top < bot) {
                 top = -1;
@@ -2085,7 +2112,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                             const uint2 mb = stk_meta[bs];
                             if (uni(try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(mb.x), uni(mb.y), slot_bytes)) == 0u) break;
                             ++bot;
-                            ++donations;
+                            tally(donations, &WorkerStats::donations, 1u);
                             moved += 2u * copy_bytes<NodeT>(w.n);
                         }
                     }
@@ -2097,7 +2124,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 have = true;
             } else {
                 if (g != kNone) {
-                    total_nodes += pending;
+                    tally(total_nodes, &WorkerStats::nodes, pending);
                     flush_nodes<STAGED>(a, gd, g, pending, moved, flush_every, true);
                     finish_unit<SERVE>(a, g, gd);
                     g = kNone;
@@ -2106,9 +2133,9 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 const uint64_t t_idle = wall_clock64();
                 Acquired q = acquire<SERVE, BITS>(a, w, slot_bytes, counted, rnd ^ (uint32_t)t_idle);
                 counted = false;
-                idle_ticks += wall_clock64() - t_idle;
+                tally(idle_ticks, &WorkerStats::idle_ticks, wall_clock64() - t_idle);
                 if (q.kind == 0) break;
-                steals += q.kind == 1;
+                if (q.kind == 1) tally(steals, &WorkerStats::steals, 1u);
                 if (q.kind == 1) {
                     g = q.g;
                 } else {
@@ -2186,7 +2213,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 continue;
             }
             if (++pending >= flush_every) {
-                total_nodes += pending;
+                tally(total_nodes, &WorkerStats::nodes, pending);
                 flush_nodes<STAGED>(a, gd, g, pending, moved, flush_every, false);
                 uint32_t stop_all = 0;
                 if (lane_id() == 0) stop_all = ld_rlx(&a.glob->cancel) || past_deadline(a);
@@ -2286,9 +2313,9 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 for (uint32_t spins = 0;; ++spins) {
                     const uint32_t bs = (uint32_t)bot % a.depth;
                     uint2 m = stk_meta[bs];
-                    if (try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(m.x), uni(m.y), slot_bytes)) {
+                    if (uni(try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(m.x), uni(m.y), slot_bytes)) != 0u) {
                         ++bot;
-                        ++donations;
+                        tally(donations, &WorkerStats::donations, 1u);
                         moved += 2u * copy_bytes<NodeT>(w.n);
                         sent = true;
                         break;
@@ -2317,7 +2344,7 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         dry = false;
         const bool donate = a.version == 1 && wants_donation<BITS>(a, ld_rlx(&a.glob->counter), rnd) != 0u;
         if (donate && top < bot && uni(try_enqueue(a, w, w.base, g, d, v, slot_bytes)) != 0u) {
-            ++donations;
+            tally(donations, &WorkerStats::donations, 1u);
             moved += copy_bytes<NodeT>(w.n);
         } else {
             const bool older = top >= bot;
@@ -2329,9 +2356,9 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
             if (donate && older) {
                 const uint32_t bs = (uint32_t)bot % a.depth;
                 uint2 m = stk_meta[bs];
-                if (try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(m.x), uni(m.y), slot_bytes)) {
+                if (uni(try_enqueue(a, w, stk + (size_t)bs * slot_bytes, g, uni(m.x), uni(m.y), slot_bytes)) != 0u) {
                     ++bot;
-                    ++donations;
+                    tally(donations, &WorkerStats::donations, 1u);
                     moved += 2u * copy_bytes<NodeT>(w.n);
                 }
             }
@@ -2340,13 +2367,17 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
         d += 1;
     }
     if (lane_id() == 0) {
-        WorkerStats ws;
-        ws.nodes = total_nodes;
-        ws.idle_ticks = idle_ticks;
-        ws.donations = donations;
-        ws.steals = steals;
-        ws.exit_tick = wall_clock64();
-        a.wstats[wid] = ws;
+        if constexpr (kTally) {
+            a.wstats[wid].exit_tick = wall_clock64();
+        } else {
+            WorkerStats ws;
+            ws.nodes = total_nodes;
+            ws.idle_ticks = idle_ticks;
+            ws.donations = donations;
+            ws.steals = steals;
+            ws.exit_tick = wall_clock64();
+            a.wstats[wid] = ws;
+        }
         if constexpr (SERVE) {
             // a server's statistics and error word live in pinned host
             // memory: stopping a server then needs no copy, which could wait
