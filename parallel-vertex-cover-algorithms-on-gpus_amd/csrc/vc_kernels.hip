@@ -1835,12 +1835,13 @@ __device__ __forceinline__ Acquired acquire(const SolveArgs &a, const N &w, uint
 // 8 x dormant_ticks they join (register and look for work) while at most
 // one in eight registered workers waits, and otherwise sleep again, for
 // max(dormant_ticks, elapsed / 8) with a jitter.  In between, every
-// dormant_ticks / 4 (jittered), they only look whether the launch is over
+// dormant_ticks / 16 (jittered), they only look whether the launch is over
 // (its own cache line, not the pool's counter) and leave if so: a search
-// that ends early then waits about dormant_ticks / 4 for them instead of up
-// to 1.5 x max(dormant_ticks, elapsed / 8).  Measured: BA n = 400 MVC
-// (29 nodes) 0.34 -> 0.22 ms, 3-regular n = 120 MVC 10-14% faster, the
-// one-graph-per-launch solve of 256 batch graphs 123 -> 128 graphs/s.  The
+// that ends early then waits about that long for them instead of up
+// to 1.5 x max(dormant_ticks, elapsed / 8).  Measured at dormant_ticks / 4: BA
+// n = 400 MVC (29 nodes) 0.34 -> 0.22 ms, 3-regular n = 120 MVC 10-14% faster,
+// the one-graph-per-launch solve of 256 batch graphs 123 -> 128 graphs/s.  One
+// wave looks for its workgroup.  The
 // join decisions keep their schedule: reading the pool's counter as often
 // as this made a 36k-node search 20% slower (contention on that line, and
 // workers joining where they only added more).  A search that runs longer
@@ -2098,9 +2099,8 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                     // offers here, one entry after the other while they are
                     // wanted.  (Not in servers, where a hard request that
                     // donates more keeps the next ones waiting: 2.4 instead of
-                    // 1.9 ms; nor in the 7-waves kernels of budgeted launches,
-                    // which have no registers left for it: a batched step took
-                    // 3.33 s instead of 2.82.)
+                    // 1.9 ms; nor in the kernels of budgeted launches: a batched
+                    // step took 3.33 s instead of 2.82, in more spills.)
                     const uint64_t now = wall_clock64();
                     if (!dry) {
                         dry = true;
@@ -2756,9 +2756,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     solve_body<int16_t, false, false, true, false>(a);
 }
 // Launches in which every graph has a node budget (searches_nodes): no bitset
-// search, so 7 waves per SIMD and 72 VGPRs (about 40 spilled, mostly off the
-// per-node path).  Per batched step: 2.87 s at 7 waves against 3.16 s at 6 (80
-// VGPRs) and 3.38 s at 8 (64 VGPRs, 68 spilled).
+// search, so 7 waves per SIMD, as many as have LDS at n = 400, and 72 VGPRs
+// without spills: 2.22 s per batched step, 2.84 with 43 spilled (solve_body).
+// (6 and 8 waves, 80 and 64 VGPRs, took 10% and 18% longer than 7 when all three
+// spilled.)
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7))) void solve_kernel_off16_nodes(SolveArgs a)
 {
     solve_body<int16_t, false, false, true, false, false, false>(a);
@@ -3360,7 +3361,7 @@ vc_status plan_launch(vc_ctx *ctx, uint32_t nmax, uint32_t depth, const vc_param
 // launch's nodes are those of graphs that end at the budget.  A node of the
 // bitset search costs much more than one of the general search, and the
 // general search runs 28 workers per CU instead of four: 4,096 graphs with a
-// budget of 2^20 nodes each take 2.8 s (2,697 solved) against 17.0 s (2,895).
+// budget of 2^20 nodes each take 2.2 s (2,697 solved) against 17.0 s (2,895).
 // So graphs with a budget are searched without it, and a launch of only such
 // graphs keeps no contexts in LDS and fills the SIMDs.
 bool searches_nodes(const vc_graphs *set, const vc_job *jobs)
@@ -3956,7 +3957,7 @@ static vc_status solve_set(vc_ctx *ctx, vc_graphs *set, const vc_job *jobs, cons
 // launch each, first the graphs with one (searches_nodes), in the time that the
 // call has.  In one launch the budgets' general search had four workers per CU
 // instead of 28: 4,095 graphs at 2^20 nodes and one without a budget took 14.4
-// s, in two launches 2.84.  Budgets of fewer than kSplitNodes nodes in all cost
+// s, in two launches 2.23.  Budgets of fewer than kSplitNodes nodes in all cost
 // less in one launch (about 5 ns more a node) than a second launch does.
 constexpr uint64_t kSplitNodes = 1u << 15;
 
@@ -4318,9 +4319,9 @@ extern "C" vc_status vc_autotune(vc_ctx *ctx, const vc_graphs *set, const vc_job
     std::vector<vc_params> cands;
     // The automatic workgroup goes first, and another shape has to be 5% faster
     // than the best before it, twice: on a sample shapes differ by less than two runs of
-    // one do (512 graphs at 2^20 nodes: 64, 128 and 256 threads 505-550 ms), and
+    // one do (512 graphs at 2^20 nodes: 64, 128 and 256 threads 409-426 ms), and
     // one picked for that can be 7% slower on the whole (4,096 graphs, 64
-    // threads: 3.04 s, 256: 2.82).
+    // threads: 2.38 s, 256: 2.22).
     uint32_t first = 256u;
     {
         vc_params p = *base;
