@@ -156,6 +156,7 @@ struct SolveArgs {
     uint32_t qthreshold;    // donate while enqueued < qthreshold
     uint32_t ring_guard;    // 1 = the ring can fill (fewer than six slots per worker)
     uint64_t offer_ticks;   // pops without a branch for this long: offer stack entries
+    uint64_t large_ticks;   // contexts of 256 vertices once the launch has run this long
     uint32_t workers;
     uint32_t version;       // 0 static split (stack only), 1 hybrid
     uint32_t start_depth;   // static split depth

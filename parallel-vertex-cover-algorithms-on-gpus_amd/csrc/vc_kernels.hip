@@ -2262,7 +2262,17 @@ __device__ __forceinline__ void solve_body(const SolveArgs &a)
                 }
                 continue;
             }
-            if (BITS && gd.max_nodes == 0u && s.live <= a.bits_max) {
+            // A launch's first 200 us take remainders of at most 128 vertices to
+            // the bitset search: the code for 256 is as large as an instruction
+            // cache, and fetching it on every CU costs a search that ends within
+            // that time more than the better bound saves.  With 0 / 100 / 200 / 300
+            // us: ER n = 500, mean degree 3.4, 0.47 / 0.34 / 0.24 / 0.24 ms (0.31
+            // without the bitset search); n = 1,000, degree 3, 0.53 / 0.53 / 0.40 /
+            // 0.33 (0.47); BA n = 1,000, m = 3, 0.39 / 0.39 / 0.32 / 0.32 (0.33);
+            // n = 400, m = 4, 0.78 / 0.77 / 0.86 / 0.92; ER n = 400, degree 4, 7.3 /
+            // 7.2 / 7.9 / 8.2 (whose parts then make contexts of their own).
+            if (BITS && gd.max_nodes == 0u && s.live <= a.bits_max &&
+                (s.live <= kBitsMaxSmall || (int64_t)(wall_clock64() - uni64(ld_rlx(&a.glob->t0))) >= (int64_t)a.large_ticks)) {
                 bits = s.live;
             } else if (s.maxdeg <= 2) {
                 // cycles only: some minimum cover holds v
@@ -3417,6 +3427,7 @@ void fill_args(SolveArgs &a, const vc_ctx *ctx, const Plan &pl, char *base, uint
                uint64_t limit_ticks)
 {
     a.offer_ticks = (uint64_t)ctx->wall_khz / 5u;  // 200 us
+    a.large_ticks = (uint64_t)ctx->wall_khz / 5u;  // 200 us
     a.off16 = pl.off16;
     a.glob = reinterpret_cast<Global *>(base + pl.off_glob);
     a.stk = base + pl.off_stk;

@@ -133,18 +133,19 @@ def _sparse_core(n):
     return np.concatenate(parts), want
 
 
-def _solve_three(ctx, n, e, want, params):
+def _solve_three(ctx, n, e, want, params, copies=1):
     """MVC, and PVC on both sides of it, on a graph whose MVC is known."""
     og = O.from_edges(n, e)
-    gs = ctx.upload([vcgpu.csr_from_edges(n, e)] * 3)
+    gs = ctx.upload([vcgpu.csr_from_edges(n, e)] * (3 * copies))
     jobs = [vcgpu.Job(vcgpu.VC_MVC, 0, n - 1, 0), vcgpu.Job(vcgpu.VC_PVC, want - 1, n - 1, 0), vcgpu.Job(vcgpu.VC_PVC, want, n - 1, 0)]
-    (mvc, no, yes), _, st = ctx.solve(gs, jobs, params)
+    res, _, st = ctx.solve(gs, jobs * copies, params)
     assert st == vcgpu.VC_OK
-    assert mvc.solved and mvc.minimum == want, (n, mvc.minimum, want)
-    assert no.solved and not no.k_found, n
-    assert yes.solved and yes.k_found, n
-    for r in (mvc, yes):
-        assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == want, n
+    for mvc, no, yes in zip(res[::3], res[1::3], res[2::3]):
+        assert mvc.solved and mvc.minimum == want, (n, mvc.minimum, want)
+        assert no.solved and not no.k_found, n
+        assert yes.solved and yes.k_found, n
+        for r in (mvc, yes):
+            assert O.cover_is_valid(og, np.asarray(r.cover, np.uint8)) and int(np.sum(r.cover)) == want, n
 
 
 @pytest.mark.parametrize("n", [127, 128, 129, 160, 191, 192, 194, 254, 255, 256, 257])
@@ -176,3 +177,34 @@ def test_remainders_of_larger_graphs_match_oracle(ctx, core, version):
         hang = [(keep[(3 * i) % core], rest[2 * i]) for i in range(pairs)] + [(rest[2 * i], rest[2 * i + 1]) for i in range(pairs)]
         full = np.concatenate([keep[np.asarray(e, np.int64)], np.asarray(hang, np.uint32)]).astype(np.uint32)
         _solve_three(ctx, n, full, want + pairs, vcgpu.Params(version=version, start_depth=2, time_limit_ms=60000))
+        if core > 128 and version == vcgpu.VC_HYBRID and (core < 200 or e is cores[0]):
+            # a launch takes remainders of more than 128 vertices to the search
+            # once it has run 200 us: four workers for 24 graphs (the large sparse
+            # cores take them a minute)
+            _solve_three(ctx, n, full, want + pairs, vcgpu.Params(num_blocks=4, block_dim=64, time_limit_ms=60000), copies=8)
+
+
+@pytest.mark.parametrize("seed", [3, 8])
+def test_small_searches_do_not_fetch_the_code_for_256(ctx, seed):
+    """150 nodes on a graph of 500 vertices: with remainders of up to 256 vertices
+    on masks from the start it took 1.5 to 2 times as long as in a workgroup of 512 threads,
+    whose contexts have at most 128."""
+    n = 500
+    p = np.random.default_rng(seed).integers(0, n, size=(1764, 2))
+    p = np.unique(np.sort(p[p[:, 0] != p[:, 1]], axis=1), axis=0)
+    e = np.random.default_rng(seed + 1).permutation(p)[:850].astype(np.uint32)
+    og = O.from_edges(n, e)
+    want, stats, _ = O.mvc(og, max_nodes=2_000_000)
+    assert stats["completed"]
+    g = vcgpu.csr_from_edges(n, e)
+    gs = ctx.upload(g)
+    job = vcgpu.Job(vcgpu.VC_MVC, 0, vcgpu.upper_bound(g, seed=1)[0], 0)
+    ms = {}
+    for block in (512, 0):
+        times = []
+        for _ in range(15):
+            (r,), info, st = ctx.solve(gs, job, vcgpu.Params(block_dim=block, time_limit_ms=60000))
+            assert st == vcgpu.VC_OK and r.solved and r.minimum == want
+            times.append(info.kernel_ms)
+        ms[block] = sorted(times)[7]
+    assert ms[0] < 1.35 * ms[512], ms
